@@ -2,7 +2,7 @@
 
 Every case is one pass through the public entry points of ``quicknn_amd.hip`` (the resident context of
 ``include/qnn_hip.h``), as the LLM engine calls them: weights resident, activations in context tensors, the
-outputs left in context tensors.  Six families, named by what the engine has in that place:
+outputs left in context tensors.  Seven families, named by what the engine has in that place:
 
 * ``mlp``        the gated MLP of a decoder in native INT4 (norm, gate/up, SwiGLU, down, residual)
 * ``gguf``       the projections of a decoder layer in mixed GGUF encodings (q, k, v, o, gate/up, GEGLU, down)
