@@ -57,39 +57,143 @@ __global__ void k_finite(const float *a, int n, int *flag) {
 
 // GO_NORM (tensor.comp:63-73), row-major rows: optional mean subtraction
 // (flags&1), x*inversesqrt(mean(x^2)+eps)*(gamma|1 [+1 if flags&4]) [+beta].
-__global__ __launch_bounds__(256) void k_norm(float *dst, const float *a, const void *gamma, int gamma_bf16,
-                                              const void *beta, int beta_bf16, int dim, int flags, int soff,
-                                              int unit_gamma, float eps) {
-  __shared__ float red[256];
-  const int row = blockIdx.x, lane = threadIdx.x;
-  const float *x = a + soff + size_t(row) * dim;
-  auto sum_group = [&](float v) {
-    red[lane] = v;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (lane < s) red[lane] += red[lane + s];
-      __syncthreads();
+//
+// A norm is one dependent chain: the row's loads, one sum (two with the mean)
+// over its threads, the stores.  So a row is held in registers: every load of
+// x, gamma and beta is issued at once (H pieces of 4 elements per thread),
+// the sum meets by a lane butterfly and, for W = 4 waves per row, one pass
+// through LDS with a single barrier.  Rows of at most 512 elements (the
+// per-head q and k norms) take one wave each, four rows per workgroup and no
+// barrier.  Longer rows than 4 * 256 * 8 take k_norm_long, which reads them
+// again for each sum.  VEC: pieces are 16-byte loads; otherwise (a row length
+// that is not a multiple of 4, or an offset that is not) one element each.
+// Before, a thread walked its elements in a loop (three loops, each load
+// waited for) between LDS trees of nine barriers: 6.8 us for one row of 2560
+// (kernel trace).  Measured: four INT4 MLP layers of 2560 -> 9728 with a norm
+// each, one token 91.1 -> 80.5 us, eight tokens 120.6 -> 101.6 us.
+struct NormArgs {
+  float *dst;
+  const float *a;
+  const void *gamma, *beta;  // null: 1, 0
+  int gamma_bf16, beta_bf16, rows, dim, flags, soff;
+  float eps;
+};
+__device__ __forceinline__ float4 load_vec4(const void *p, int bf16, int j) {  // elements j..j+3, j % 4 == 0
+  if (!bf16) return *reinterpret_cast<const float4 *>(static_cast<const float *>(p) + j);
+  const uint2 v = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(p) + j);
+  return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u), __uint_as_float(v.y << 16),
+                     __uint_as_float(v.y & 0xFFFF0000u));
+}
+template <int W, int H, bool VEC>
+__global__ __launch_bounds__(256) void k_norm(const NormArgs a) {
+  static_assert(W == 1 || W == 4, "waves per row");
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row = W == 4 ? blockIdx.x : blockIdx.x * 4 + wave;
+  if (W == 1 && row >= a.rows) return;  // whole waves; no barrier below
+  const int t = W == 4 ? int(threadIdx.x) : lane, dim = a.dim;
+  const float *x = a.a + a.soff + size_t(row) * dim;
+  const bool sub = (a.flags & 1) != 0, gam = a.gamma != nullptr, bet = a.beta != nullptr;
+  auto load = [&](const void *p, int bf16, int j) {
+    if (VEC) return load_vec4(p, bf16, j);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    v.x = load_vec(p, bf16, j);
+    if (j + 1 < dim) v.y = load_vec(p, bf16, j + 1);
+    if (j + 2 < dim) v.z = load_vec(p, bf16, j + 2);
+    if (j + 3 < dim) v.w = load_vec(p, bf16, j + 3);
+    return v;
+  };
+  float4 xv[H], gv[H], bv[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const int j = 4 * (t + 64 * W * h);
+    xv[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (j < dim) xv[h] = load(x, 0, j);
+  }
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const int j = 4 * (t + 64 * W * h);
+    gv[h] = make_float4(1.f, 1.f, 1.f, 1.f);
+    bv[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (j < dim) {
+      if (gam) gv[h] = load(a.gamma, a.gamma_bf16, j);
+      if (bet) bv[h] = load(a.beta, a.beta_bf16, j);
     }
-    float r = red[0];
+  }
+  __shared__ float red[2][4];
+  auto sum_row = [&](float v, int slot) {
+    v = dev::wave_sum_xor(v);
+    if constexpr (W == 4) {
+      if (lane == 0) red[slot][wave] = v;
+      __syncthreads();
+      v = (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
+    }
+    return v;
+  };
+  if (sub) {
+    float part = 0.0f;
+#pragma unroll
+    for (int h = 0; h < H; ++h) part += (xv[h].x + xv[h].y) + (xv[h].z + xv[h].w);
+    const float mean = sum_row(part, 0) / float(dim);
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int j = 4 * (t + 64 * W * h);  // elements past the row stay zero
+      if (j < dim) xv[h].x -= mean;
+      if (j + 1 < dim) xv[h].y -= mean;
+      if (j + 2 < dim) xv[h].z -= mean;
+      if (j + 3 < dim) xv[h].w -= mean;
+    }
+  }
+  float part = 0.0f;
+#pragma unroll
+  for (int h = 0; h < H; ++h)
+    part += (xv[h].x * xv[h].x + xv[h].y * xv[h].y) + (xv[h].z * xv[h].z + xv[h].w * xv[h].w);
+  const float inv = rsqrtf(sum_row(part, 1) / float(dim) + a.eps);
+  const float one = (a.flags & 4) ? 1.0f : 0.0f;
+  float *o = a.dst + a.soff + size_t(row) * dim;
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const int j = 4 * (t + 64 * W * h);
+    if (j >= dim) continue;
+    const float4 v = make_float4(xv[h].x * inv * (gv[h].x + one) + bv[h].x, xv[h].y * inv * (gv[h].y + one) + bv[h].y,
+                                 xv[h].z * inv * (gv[h].z + one) + bv[h].z, xv[h].w * inv * (gv[h].w + one) + bv[h].w);
+    if (VEC) {
+      *reinterpret_cast<float4 *>(o + j) = v;
+    } else {
+      o[j] = v.x;
+      if (j + 1 < dim) o[j + 1] = v.y;
+      if (j + 2 < dim) o[j + 2] = v.z;
+      if (j + 3 < dim) o[j + 3] = v.w;
+    }
+  }
+}
+
+// Rows of any length, read once per sum and once for the values.
+__global__ __launch_bounds__(256) void k_norm_long(const NormArgs a) {
+  __shared__ float red[2][4];
+  const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, dim = a.dim;
+  const float *x = a.a + a.soff + size_t(row) * dim;
+  auto sum_row = [&](float v, int slot) {
+    v = dev::wave_sum_xor(v);
+    if (lane == 0) red[slot][wave] = v;
     __syncthreads();
-    return r;
+    return (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
   };
   float mean = 0.0f, part = 0.0f;
-  if (flags & 1) {
-    for (int j = lane; j < dim; j += 256) part += x[j];
-    mean = sum_group(part) / float(dim);
+  if (a.flags & 1) {
+    for (int j = threadIdx.x; j < dim; j += 256) part += x[j];
+    mean = sum_row(part, 0) / float(dim);
+    part = 0.0f;
   }
-  part = 0.0f;
-  for (int j = lane; j < dim; j += 256) {
-    float v = x[j] - mean;
+  for (int j = threadIdx.x; j < dim; j += 256) {
+    const float v = x[j] - mean;
     part += v * v;
   }
-  const float squares = sum_group(part);
-  const float inv = rsqrtf(squares / float(dim) + eps);
-  for (int j = lane; j < dim; j += 256) {
-    float scale = (unit_gamma ? 1.0f : load_vec(gamma, gamma_bf16, j)) + ((flags & 4) ? 1.0f : 0.0f);
-    float b = ((flags & 1) && !(flags & 8) && beta) ? load_vec(beta, beta_bf16, j) : 0.0f;
-    dst[soff + size_t(row) * dim + j] = (x[j] - mean) * inv * scale + b;
+  const float inv = rsqrtf(sum_row(part, 1) / float(dim) + a.eps);
+  const float one = (a.flags & 4) ? 1.0f : 0.0f;
+  for (int j = threadIdx.x; j < dim; j += 256) {
+    const float scale = (a.gamma ? load_vec(a.gamma, a.gamma_bf16, j) : 1.0f) + one;
+    const float b = a.beta ? load_vec(a.beta, a.beta_bf16, j) : 0.0f;
+    a.dst[a.soff + size_t(row) * dim + j] = (x[j] - mean) * inv * scale + b;
   }
 }
 
@@ -297,8 +401,34 @@ void misc_finite(const float *a, int n, int *flag, hipStream_t s) {
 }
 void misc_norm(float *dst, const float *a, const void *gamma, int gamma_bf16, const void *beta, int beta_bf16,
                int rows, int dim, int flags, int src_off, int unit_gamma, float eps, hipStream_t s) {
-  hipLaunchKernelGGL(k_norm, dim3(rows), dim3(256), 0, s, dst, a, gamma, gamma_bf16, beta, beta_bf16, dim, flags,
-                     src_off, unit_gamma, eps);
+  NormArgs n;
+  n.dst = dst;
+  n.a = a;
+  n.gamma = unit_gamma ? nullptr : gamma;
+  n.beta = (flags & 1) && !(flags & 8) ? beta : nullptr;
+  n.gamma_bf16 = gamma_bf16;
+  n.beta_bf16 = beta_bf16;
+  n.rows = rows;
+  n.dim = dim;
+  n.flags = flags;
+  n.soff = src_off;
+  n.eps = eps;
+  // 16-byte pieces: every row, and gamma and beta (8-byte pieces in bf16), start aligned.
+  auto aligned = [](const void *p, int bf16) { return !p || reinterpret_cast<uintptr_t>(p) % (bf16 ? 8 : 16) == 0; };
+  const bool vec = dim % 4 == 0 && src_off % 4 == 0 && aligned(dst, 0) && aligned(a, 0) &&
+                   aligned(n.gamma, gamma_bf16) && aligned(n.beta, beta_bf16);
+#define QNN_NORM(W, H)                                                                             \
+  do {                                                                                             \
+    const dim3 grid(W == 4 ? rows : (rows + 3) / 4);                                               \
+    if (vec) hipLaunchKernelGGL((k_norm<W, H, true>), grid, dim3(256), 0, s, n);                   \
+    else hipLaunchKernelGGL((k_norm<W, H, false>), grid, dim3(256), 0, s, n);                      \
+  } while (0)
+  if (dim <= 256) QNN_NORM(1, 1);
+  else if (dim <= 512) QNN_NORM(1, 2);
+  else if (dim <= 4096) QNN_NORM(4, 4);
+  else if (dim <= 8192) QNN_NORM(4, 8);
+  else hipLaunchKernelGGL(k_norm_long, dim3(rows), dim3(256), 0, s, n);
+#undef QNN_NORM
   hip_check(hipGetLastError(), "norm");
 }
 void misc_moe_route(float *routes, const float *logits, int rows, int experts, int k, int normalize,

@@ -319,3 +319,43 @@ def test_graph_replays_gguf_projections_and_attention_match_eager(ctx, rng):
                                 oracle.cpu_linear(w4b, oracle.ENC_Q4_K, x0[2][r * k:(r + 1) * k], k, n)) <= 1e-3
     for t in xs + ys + [q, o, other, cache]:
         ctx.Recycle(t)
+
+
+@pytest.mark.parametrize("dim", [1, 3, 64, 128, 255, 256, 257, 512, 513, 1000, 2560, 4095, 4096, 4097, 8192, 8195])
+@pytest.mark.parametrize("rows,soff,flags,gamma_kind", [(1, 0, 0, "f32"), (5, 4, 4, "bf16"), (6, 3, 1, "f32"),
+                                                        (3, 0, 1 | 8, "unit")])
+def test_norm_row_lengths(ctx, rng, rows, soff, flags, gamma_kind, dim):
+    """Every launch shape of GO_NORM: one wave per row, four, the long-row loop; 16-byte and single-element
+    loads (odd lengths and offsets); nothing outside the rows is written.  An fp32 sum of dim squares in any
+    order is off by less than dim / 2 ulp, in these chunked orders by a few: 2e-6 normwise."""
+    from quicknn_amd import hip
+
+    x = (rng.standard_normal(soff + rows * dim) + 0.5).astype(np.float32)
+    gamma = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    beta = rng.standard_normal(dim).astype(np.float32)
+    g64 = gamma.astype(np.float64)
+    gb = hip.MemoryBlock(gamma, (dim,), hip.DT_F32)
+    if gamma_kind == "bf16":
+        bits = bf16_bits(gamma)
+        gb, g64 = hip.MemoryBlock(bits, (dim,), hip.DT_BF16), bf16_to_f32(bits).astype(np.float64)
+    unit = int(gamma_kind == "unit")
+    if unit:
+        g64 = np.ones(dim)
+    if flags & 4:
+        g64 = g64 + 1
+    xt, out = ctx.UploadRaw(x), ctx.UploadRaw(np.full(soff + rows * dim + 8, 7.0, np.float32))
+    ctx.KernelWeights(hip.GO_NORM, rows * dim, out, xt, None if unit else gb,
+                      hip.MemoryBlock(beta, (dim,), hip.DT_F32) if flags & 1 and not flags & 8 else None,
+                      [rows, dim, flags, 0, 0, soff, unit, f32_bits(1e-5)])
+    got = ctx.Download(out)
+    v = x[soff:].reshape(rows, dim).astype(np.float64)
+    if flags & 1:
+        v = v - v.mean(axis=1, keepdims=True)
+    want = v / np.sqrt((v ** 2).mean(axis=1, keepdims=True) + np.float32(1e-5)) * g64
+    if flags & 1 and not flags & 8:
+        want = want + beta
+    assert np.all(got[:soff] == 7.0) and np.all(got[soff + rows * dim:] == 7.0)
+    if dim > 1 or not flags & 1:  # a centred row of one element is the beta alone
+        assert normwise_rel_err(got[soff:soff + rows * dim].reshape(rows, dim), want) < 2e-6
+    ctx.Recycle(xt)
+    ctx.Recycle(out)
