@@ -12,11 +12,7 @@
 //   activations, two pieces in flight per iteration, then a butterfly sum.
 // * fused gate/up SwiGLU, one row (dense_swiglu_launch, op 66): as the
 //   matvec, with the gate and up rows of an output read in the same pass.
-// * several rows (dense_gemm_launch): a 256-thread workgroup computes a tile
-//   of 64 outputs x 16 rows; 32-wide K slices of the weight tile and the
-//   activation tile are staged in LDS (weights padded to 33 floats per row so
-//   the 64 lanes of a wave read 64 different banks), and each thread
-//   accumulates 4 rows of one output.
+// * several rows (dense_gemm_launch): fp32 matrix cores (k_dense_mm).
 #include "qnn_internal.h"
 #include "qnn_lanes.h"
 
@@ -160,50 +156,92 @@ __global__ __launch_bounds__(256) void k_dense_swiglu(const void *__restrict__ w
   }
 }
 
-constexpr int kTN = 64, kTM = 16, kTK = 32;
+// ---- several rows: fp32 matrix cores ------------------------------------------
+// Y[m][n] = sum_k X[m][k] W[n][k] on v_mfma_f32_16x16x4_f32: fp32 products
+// and sums, as the VALU's, at twice its rate and with no LDS staging.  Lane l
+// of a wave holds elements 8q .. 8q+7 (q = l / 16) of a 32-element K-step of
+// row l % 16 of X and of W, and MFMA i of the step takes element i of both:
+// the same permutation of k on both sides.  A wave computes 16 TM x 16 TN of
+// Y, and the KW waves of a workgroup take the K-steps in turn, requesting the
+// next step's pieces before the current step's products, and meet in LDS in
+// wave order.  The work is small and its chain long (the router: 128 x 128
+// outputs over 2048 elements), so what bounds it is the latency of a wave's
+// few loads: small outputs take 16 waves per 16 x 16 tile (64 workgroups of 4
+// steps per wave at the router's shape), larger ones 32 x 32 tiles, where a
+// loaded piece feeds two products, with fewer waves per tile.
+// Measured (kernel trace, bf16 router of 128 experts, 128 rows of 2048): a
+// tile of 64 x 16 outputs per workgroup with LDS-staged scalar products took
+// 189.6 us (16 workgroups, 64 barriers), this 7.6 us.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <bool BF16>
-__global__ __launch_bounds__(256) void k_dense_gemm(const void *__restrict__ w, const float *__restrict__ x,
-                                                    float *__restrict__ y, int m, int n, int k) {
-  __shared__ float ws[kTN][kTK + 1];
-  __shared__ float xs[kTM][kTK];
-  const int t = threadIdx.x;
-  const int n0 = blockIdx.x * kTN, m0 = blockIdx.y * kTM;
-  const int nl = t & 63, mg = t >> 6;  // output n0 + nl, rows m0 + 4*mg .. +3
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < k; k0 += kTK) {
+template <bool BF16, bool VEC>
+__device__ __forceinline__ void load_step(float (&v)[8], const void *base, size_t row, int k, int j) {
 #pragma unroll
-    for (int i = 0; i < kTN * kTK / 256; ++i) {  // weight tile: 8 elements per thread
-      const int e = i * 256 + t, r = e / kTK, c = e % kTK;
-      const int gn = n0 + r, gk = k0 + c;
-      float v = 0.0f;
-      if (gn < n && gk < k)
-        v = BF16 ? bf16_to_f32(static_cast<const uint16_t *>(w)[size_t(gn) * k + gk])
-                 : static_cast<const float *>(w)[size_t(gn) * k + gk];
-      ws[r][c] = v;
-    }
+  for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+  if constexpr (VEC) {  // k % 8 == 0: the lane's 8 elements are all inside the row or all past it
+    if (j < k) load8<BF16>(static_cast<const uint8_t *>(base) + row * size_t(k) * (BF16 ? 2 : 4), j, v);
+  } else {
 #pragma unroll
-    for (int i = 0; i < kTM * kTK / 256; ++i) {  // activation tile: 2 elements per thread
-      const int e = i * 256 + t, r = e / kTK, c = e % kTK;
-      const int gm = m0 + r, gk = k0 + c;
-      xs[r][c] = gm < m && gk < k ? x[size_t(gm) * k + gk] : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (int c = 0; c < kTK; ++c) {
-      const float wv = ws[nl][c];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = fmaf(wv, xs[4 * mg + i][c], acc[i]);
-    }
-    __syncthreads();
+    for (int i = 0; i < 8; ++i)
+      if (j + i < k) v[i] = weight_at<BF16>(base, row * size_t(k) + j + i);
   }
-  const int gn = n0 + nl;
-  if (gn < n) {
+}
+
+template <bool BF16, bool VEC, int TM, int TN, int KW>
+__global__ __launch_bounds__(64 * KW) void k_dense_mm(const void *__restrict__ w, const float *__restrict__ x,
+                                                      float *__restrict__ y, int m, int n, int k) {
+  __shared__ float red[KW][TM * TN * 4][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int n0 = blockIdx.x * 16 * TN, m0 = blockIdx.y * 16 * TM;
+  size_t xr[TM], wr[TN];  // rows past the end read the last one; their outputs are not written
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int gm = m0 + 4 * mg + i;
-      if (gm < m) y[size_t(gm) * n + gn] = acc[i];
-    }
+  for (int i = 0; i < TM; ++i) xr[i] = size_t(min(m0 + 16 * i + r, m - 1));
+#pragma unroll
+  for (int i = 0; i < TN; ++i) wr[i] = size_t(min(n0 + 16 * i + r, n - 1));
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float xa[2][TM][8], wa[2][TN][8];
+  auto load = [&](int s, int k0) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) load_step<false, VEC>(xa[s][i], x, xr[i], k, k0 + 8 * q);
+#pragma unroll
+    for (int i = 0; i < TN; ++i) load_step<BF16, VEC>(wa[s][i], w, wr[i], k, k0 + 8 * q);
+  };
+  auto products = [&](int s) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[s][i][e], wa[s][j][e], acc[i][j], 0, 0, 0);
+  };
+  int k0 = wave * 32;
+  if (k0 < k) load(0, k0);
+  for (; k0 < k; k0 += 64 * KW) {  // two steps per turn, so that the stages are indexed statically
+    const int k1 = k0 + 32 * KW, k2 = k0 + 64 * KW;
+    if (k1 < k) load(1, k1);
+    products(0);
+    if (k2 < k) load(0, k2);
+    if (k1 < k) products(1);
+  }
+  // Lane l holds rows 4q .. 4q+3 of column r of each 16 x 16 tile.
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[wave][(i * TN + j) * 4 + e][lane] = acc[i][j][e];
+  __syncthreads();
+  for (int o = wave; o < TM * TN * 4; o += KW) {
+    float v = 0.0f;
+#pragma unroll
+    for (int p = 0; p < KW; ++p) v += red[p][o][lane];
+    const int tile = o >> 2, row = m0 + 16 * (tile / TN) + 4 * q + (o & 3), col = n0 + 16 * (tile % TN) + r;
+    if (row < m && col < n) y[size_t(row) * n + col] = v;
   }
 }
 
@@ -243,9 +281,26 @@ void dense_swiglu_launch(const void *wg, int bg, const void *wu, int bu, const f
 }
 
 void dense_gemm_launch(const void *w, int bf16, const float *x, float *y, int m, int n, int k, hipStream_t s) {
-  const dim3 grid((n + kTN - 1) / kTN, (m + kTM - 1) / kTM), block(256);
-  if (bf16) hipLaunchKernelGGL(k_dense_gemm<true>, grid, block, 0, s, w, x, y, m, n, k);
-  else hipLaunchKernelGGL(k_dense_gemm<false>, grid, block, 0, s, w, x, y, m, n, k);
+  // 16-byte pieces of both operands: whole 8-element chunks, aligned rows.
+  const bool vec = k % 8 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  // 32 x 32 tiles where they still give a workgroup for every second CU, with
+  // more waves per tile while there are fewer than two per CU.
+  auto tiles = [&](int t) { return (long long)((m + t - 1) / t) * ((n + t - 1) / t); };
+#define QNN_DENSE_MM(TM, TN, KW)                                                                              \
+  do {                                                                                                        \
+    const dim3 grid((n + 16 * TN - 1) / (16 * TN), (m + 16 * TM - 1) / (16 * TM)), block(64 * KW);            \
+    if (bf16) {                                                                                               \
+      if (vec) hipLaunchKernelGGL((k_dense_mm<true, true, TM, TN, KW>), grid, block, 0, s, w, x, y, m, n, k); \
+      else hipLaunchKernelGGL((k_dense_mm<true, false, TM, TN, KW>), grid, block, 0, s, w, x, y, m, n, k);    \
+    } else {                                                                                                  \
+      if (vec) hipLaunchKernelGGL((k_dense_mm<false, true, TM, TN, KW>), grid, block, 0, s, w, x, y, m, n, k); \
+      else hipLaunchKernelGGL((k_dense_mm<false, false, TM, TN, KW>), grid, block, 0, s, w, x, y, m, n, k);   \
+    }                                                                                                         \
+  } while (0)
+  if (tiles(32) >= 512) QNN_DENSE_MM(2, 2, 4);
+  else if (tiles(32) >= 128) QNN_DENSE_MM(2, 2, 8);
+  else QNN_DENSE_MM(1, 1, 16);
+#undef QNN_DENSE_MM
   hip_check(hipGetLastError(), "dense gemm launch");
 }
 

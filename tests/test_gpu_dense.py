@@ -83,3 +83,22 @@ def test_dense_argument_errors(ctx, rng):
         ctx.VectorLinear(ctx.NewTensor(65), src, w, 64, 65)
     with pytest.raises(hip.ENotSupportedException):  # native INT4 goes through Int4Linear
         ctx.Linear(dst, src, packed, None, None, 1, 64, 64)
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("rows,n,k", [(2, 1, 1), (15, 17, 31), (16, 16, 32), (17, 33, 40), (33, 31, 513), (128, 600, 72),
+                                      (260, 516, 96), (500, 1100, 24), (512, 1056, 30)])
+def test_linear_dense_tiles(ctx, rng, bf16, rows, n, k):
+    """Every tile of the multi-row kernel (16 x 16 and 32 x 32, 4 to 16 waves), edges and remainders of each
+    dimension, 16-byte and single-element loads: the outputs and nothing else are written.  fp32 products and
+    sums: below k * 2^-24 of the sum of the products' magnitudes, whatever the order."""
+    w, w64 = weight(rng, n, k, bf16)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    src, dst = ctx.UploadRaw(x), ctx.UploadRaw(np.full(rows * n + 64, 7.0, np.float32))
+    ctx.Linear(dst, src, w, None, None, rows, k, n)
+    got = ctx.Download(dst)
+    assert np.all(got[rows * n:] == 7.0)
+    bound = (np.abs(x).astype(np.float64) @ np.abs(w64).T) * (k + 32) * 2.0 ** -24
+    assert np.all(np.abs(got[:rows * n].reshape(rows, n) - x.astype(np.float64) @ w64.T) <= bound)
+    ctx.Recycle(src)
+    ctx.Recycle(dst)
