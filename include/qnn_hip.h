@@ -287,6 +287,8 @@ int qnn_vector_linear(qnn_ctx *ctx, qnn_tensor *dst, qnn_tensor *src, const qnn_
 
 /* Int4Linear (Context.API.inc:138-142, Implementation.inc:1080-1135):
  * 1 <= rows <= 128; weight U8/NATIVE [out_dim, Int4RowBytes(in_dim)], offset 0.
+ * From 25 rows the call runs as a GEMM over two fp16 planes of the
+ * activations (weights exact), below as a matvec of up to 16 rows per pass.
  * A multi-row call may be recorded and launched with the next call: two on
  * the same input followed by QNN_GO_SWIGLU of their outputs (the engine's
  * multi-row MLP) run as one gate/up SwiGLU launch that also writes both

@@ -172,6 +172,7 @@ void reload_tuning() {
   t.gg_bw = env_int("QNN_GG_BW", t.gg_bw);
   t.gg_mt = env_int("QNN_GG_MT", t.gg_mt);
   t.i4_mfma = env_int("QNN_I4_MFMA", t.i4_mfma);
+  t.i4_gemm_rows = env_int("QNN_I4_GEMM_ROWS", t.i4_gemm_rows);
   t.i4_lanes = env_int("QNN_I4_LANES", t.i4_lanes);
   t.i4_tpw = env_int("QNN_I4_TPW", t.i4_tpw);
   t.i4_target_waves = env_int("QNN_I4_TARGET_WAVES", t.i4_target_waves);
@@ -652,17 +653,57 @@ struct OpPins {
 };
 
 // ---------------------------------------------------------------- INT4 projection
-// Caller-provided split-K workspace (the no-allocation entry point's static
-// scratch): its tickets are cleared by a fill kernel before every launch.
+// Caller-provided workspace (the no-allocation entry point's static scratch):
+// its tickets are cleared by a fill kernel before every launch.
 struct FixedWs {
   float *partial = nullptr;
   unsigned *counters = nullptr;
 };
 
+// All rows against every weight once (qnn_int4_gemm.hip).  Rows that do not
+// fit a fixed workspace together run in halves; a row's result is the same.
+void run_int4_gemm(qnn_ctx_s *ctx, I4Launch a, const FixedWs *fixed) {
+  const bool pair = a.mode == I4_SWIGLU;
+  const int rows = a.m;
+  int chunk = rows;
+  if (fixed)
+    while (chunk > 1 && int4_gemm_bytes(int4_gemm_plan(a.l, chunk), pair) > kNoAllocPartialBytes) chunk = (chunk + 1) / 2;
+  const I4Launch all = a;
+  for (int r0 = 0; r0 < rows; r0 += chunk) {
+    a.m = std::min(chunk, rows - r0);
+    a.x = all.x + size_t(r0) * all.x_stride;
+    a.y = all.y + size_t(r0) * all.y_stride;
+    if (all.g_out) {
+      a.g_out = all.g_out + size_t(r0) * all.y_stride;
+      a.u_out = all.u_out + size_t(r0) * all.y_stride;
+    }
+    const I4GemmPlan p = int4_gemm_plan(a.l, a.m);
+    uint8_t *ws = fixed ? reinterpret_cast<uint8_t *>(fixed->partial)
+                        : static_cast<uint8_t *>(ensure_work(ctx, int4_gemm_bytes(p, pair)));
+    int4_gemm_launch(a, p, ws, ctx->stream);
+  }
+}
+
 void run_int4(qnn_ctx_s *ctx, const WeightEntry *w, const WeightEntry *w2, int mode, const float *x, float *y,
               int rows, int in_dim, int out_dim, const float *prob, float *g_out = nullptr, float *u_out = nullptr,
               const FixedWs *fixed = nullptr) {
   const I4Layout &l = w->i4;
+  if (mode != I4_ACCUM && int4_gemm_applies(l, rows)) {
+    I4Launch a;
+    a.l = l;
+    a.nib = w->dptr;
+    a.nib2 = w2 ? w2->dptr : nullptr;
+    a.x = x;
+    a.x_stride = a.k = in_dim;
+    a.y = y;
+    a.y_stride = a.n = out_dim;
+    a.m = rows;
+    a.mode = mode;
+    a.g_out = g_out;
+    a.u_out = u_out;
+    run_int4_gemm(ctx, a, fixed);
+    return;
+  }
   // The kernels read activation rows as aligned 4-float pieces: a row length
   // that is not a multiple of 4 goes through a zero-padded copy.
   int k = in_dim;
@@ -847,7 +888,9 @@ bool mlp_fusion_enabled() { return tuning().fuse_mlp != 0; }
 // A gate/up SwiGLU launch gives each row the sums the two I4_STORE launches
 // would (same steps per wave, slices and parts for every 16-row chunk), so
 // the recorded triple stays bit-identical to the separate operations.
+// (The many-row GEMM's plan is the same for both.)
 bool glu_plans_match(const I4Layout &l, int rows) {
+  if (int4_gemm_applies(l, rows)) return true;
   for (int r0 = 0; r0 < rows; r0 += 16) {
     const int m = std::min(16, rows - r0);
     const I4Plan a = int4_plan(l, m, I4_STORE), b = int4_plan(l, m, I4_SWIGLU);
@@ -1434,18 +1477,26 @@ int qnn_int4_linear(qnn_ctx *ctx, qnn_tensor *dst, qnn_tensor *src, const qnn_we
                          dst->ptr != p.h && try_fused_mlp(ctx, e, dst->ptr);
       // Several rows: recorded to meet a following GO_SWIGLU (gate, up).
       qnn_ctx_s::PendingRows &q = ctx->prows;
-      if (!fused && rows >= 2 && !ctx->capturing && mlp_fusion_enabled() && in_dim % 4 == 0 &&
+      const bool gemm = int4_gemm_applies(e->i4, rows);
+      if (!fused && rows >= 2 && !ctx->capturing && mlp_fusion_enabled() && (gemm || in_dim % 4 == 0) &&
           glu_plans_match(e->i4, rows)) {
         // Sized now (its own launch and the gate/up SwiGLU launch it may join),
         // so that launching it never allocates.
-        size_t pf = 0, nc = 0;
-        for (int r0 = 0; r0 < rows; r0 += 16) {
-          const I4Plan a = int4_plan(e->i4, std::min(16, rows - r0), I4_STORE);
-          const I4Plan b = int4_plan(e->i4, std::min(16, rows - r0), I4_SWIGLU);
-          pf = std::max({pf, a.partial_floats, b.partial_floats});
-          nc = std::max({nc, a.counters, b.counters});
+        if (gemm) {
+          // A call recorded before this one was sized for its own launch:
+          // growing the workspace waits for queued work only, and recorded
+          // calls keep no pointer into it.
+          ensure_work(ctx, int4_gemm_bytes(int4_gemm_plan(e->i4, rows), true));
+        } else {
+          size_t pf = 0, nc = 0;
+          for (int r0 = 0; r0 < rows; r0 += 16) {
+            const I4Plan a = int4_plan(e->i4, std::min(16, rows - r0), I4_STORE);
+            const I4Plan b = int4_plan(e->i4, std::min(16, rows - r0), I4_SWIGLU);
+            pf = std::max({pf, a.partial_floats, b.partial_floats});
+            nc = std::max({nc, a.counters, b.counters});
+          }
+          ensure_splitk(ctx, pf, nc);
         }
-        ensure_splitk(ctx, pf, nc);
         if (q.count == 1 && q.x == src->ptr && q.rows == rows && q.in == in_dim && q.out == out_dim &&
             dst->ptr != q.y[0] && e->i4.rows == q.e[0]->i4.rows && e->i4.cols == q.e[0]->i4.cols &&
             e->i4.lanes == q.e[0]->i4.lanes) {

@@ -52,6 +52,7 @@ struct Tuning {
   int gg_bw = 0;             // QNN_GG_BW: GGUF units per wave (1 or 2)
   int gg_mt = 1;             // QNN_GG_MT: GGUF Linear below the GEMM, up to 8 rows per pass (0: one per row)
   int i4_mfma = 1;           // QNN_I4_MFMA: multi-token INT4 dot on the int8 matrix cores
+  int i4_gemm_rows = 25;     // QNN_I4_GEMM_ROWS: rows from which Int4Linear runs as a GEMM (0: never)
   int i4_lanes = 0;          // QNN_I4_LANES: lanes per INT4 row at upload (1..16)
   int i4_tpw = 1;            // QNN_I4_TPW: INT4 tiles per workgroup (1, 2, 4)
   int i4_target_waves = 0;   // QNN_I4_TARGET_WAVES: wave target of the INT4 planner
@@ -186,6 +187,24 @@ void int4_matvec_launch(const I4Launch &a, const I4Plan &p, hipStream_t s);
 void int4_repack_launch(const uint8_t *src, const I4Layout &l, void *dst, hipStream_t s);
 // one_lane: one lane per row whatever QNN_I4_LANES says (the MoE expert kernels assume it).
 I4Layout int4_layout(int rows, int cols, bool one_lane = false);
+// Many rows (qnn_int4_gemm.hip): every weight read once per call.  A row's
+// result depends on the matrix alone, not on the call's other rows, its mode
+// or its chunking.  Workspace: int4_gemm_bytes.  At most kI4GemmMaxGroups
+// groups per row: eight rows of any such call fit the no-allocation scratch.
+constexpr int kI4GemmMaxGroups = 640;
+constexpr size_t kI4GemmExpBytes = 512;  // 128 row exponents
+struct I4GemmPlan {
+  int gpad = 0, ktiles = 0, slices = 1;
+  size_t frag_bytes = 0;
+  size_t part_bytes = 0;  // per matrix
+};
+bool int4_gemm_applies(const I4Layout &l, int rows);
+I4GemmPlan int4_gemm_plan(const I4Layout &l, int rows);
+inline size_t int4_gemm_bytes(const I4GemmPlan &p, bool pair) {
+  return kI4GemmExpBytes + p.frag_bytes + p.part_bytes * (pair ? 2 : 1);
+}
+// a: as for int4_matvec_launch with all rows (m <= 128), any row length and alignment; I4_STORE or I4_SWIGLU.
+void int4_gemm_launch(const I4Launch &a, const I4GemmPlan &p, uint8_t *ws, hipStream_t s);
 void int4_dequant_launch(const I4Layout &l, const void *w, float *out, hipStream_t s);
 
 void misc_fill(float *dst, int n, uint32_t bits, hipStream_t s);

@@ -302,3 +302,35 @@ def test_sixteen_token_chunks_on_matrix_cores(ctx, rng):
         assert normwise_rel_err(got16[r], oracle.cpu_linear(p, oracle.ENC_INT4, x[r], k, n)) <= TOL, r
     ctx.Recycle(src)
     ctx.Recycle(dst)
+
+
+@pytest.mark.parametrize("rows", [25, 32, 33, 64, 65, 100, 128])
+@pytest.mark.parametrize("n,k", [(64, 32), (1, 1), (65, 33), (128, 64), (200, 96), (190, 1001), (1000, 2560), (320, 330),
+                                 (9728, 2560)])
+def test_many_rows_gemm(ctx, rng, rows, n, k):
+    """From 25 rows Int4Linear runs as a GEMM over two fp16 planes of the activations: every row tile, an odd
+    number of weight blocks and of groups, K-slices, row lengths that are no multiple of 4 or 32.  hi + lo hold
+    22 bits of each activation (above 2^-27 of its row's largest), so against the packed weights' values in
+    64 bits an output is off by 2^-21 of the products' magnitudes, by the fp32 sums (64 products a group, then
+    the groups) and by the smallest step of lo, 2^-38 of the row's largest per weight."""
+    p = make_int4(rng, n, k)
+    w = hip.MemoryBlock.int4(p)
+    x = (rng.standard_normal((rows, k)) * np.exp2(rng.integers(-20, 20, (rows, 1)))).astype(np.float32)
+    src, dst = ctx.UploadRaw(x), ctx.UploadRaw(np.full(rows * n + 64, 7.0, np.float32))
+    ctx.Int4Linear(dst, src, w, rows, k, n)
+    got = ctx.Download(dst)
+    assert np.all(got[rows * n:] == 7.0)
+    w64 = oracle.int4_dequant(p, k).astype(np.float64)
+    x64 = x.astype(np.float64)
+    bound = (np.abs(x64) @ np.abs(w64).T) * (2.0 ** -21 + (64 + k / 32) * 2.0 ** -24)
+    bound += np.abs(x64).max(1)[:, None] * 2.0 ** -38 * np.abs(w64).sum(1)
+    assert np.all(np.abs(got[:rows * n].reshape(rows, n) - x64 @ w64.T) <= bound)
+    # rows do not depend on the call they are part of
+    few, half = ctx.UploadRaw(x[rows - 25:]), ctx.NewTensor(25 * n)
+    ctx.Int4Linear(half, few, w, 25, k, n)
+    assert np.array_equal(ctx.Download(half).view(np.uint32), got[(rows - 25) * n:rows * n].view(np.uint32))
+    if k % 4 == 0:  # the fixed scratch may hold the rows in several parts only
+        ctx.Int4LinearNoAlloc(dst, src, w, rows, k, n)
+        assert np.array_equal(ctx.Download(dst).view(np.uint32), got.view(np.uint32))
+    for t in (src, dst, few, half):
+        ctx.Recycle(t)

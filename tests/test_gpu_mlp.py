@@ -224,3 +224,30 @@ def test_multi_row_triple_under_graph_capture(ctx, rng):
             assert np.array_equal(a, b), (rep, nm)
     for t in (x, g8, u8, hh):
         ctx.Recycle(t)
+
+
+@pytest.mark.parametrize("rows,hidden,inter,into", [(25, 512, 1536, "new"), (128, 2560, 9728, "new"), (100, 330, 321, "gate"),
+                                                    (70, 256, 96, "up"), (65, 1000, 64, "new")])
+def test_many_rows_pair_equals_separate(ctx, rng, tune, rows, hidden, inter, into):
+    """From 25 rows gate, up and GO_SWIGLU run as one GEMM pair: both outputs and the GLU (also written over the
+    gate or the up sums) are bit-identical to the three separate operations."""
+    from quicknn_amd import hip
+
+    g, u = hip.MemoryBlock.int4(rand_int4(rng, inter, hidden)), hip.MemoryBlock.int4(rand_int4(rng, inter, hidden))
+    x = ctx.UploadRaw(rng.standard_normal((rows, hidden)).astype(np.float32))
+    got = {}
+    for fuse in ("1", "0"):
+        tune("QNN_FUSE_MLP", fuse)
+        gt, ut, ht = (ctx.NewTensor(rows * inter) for _ in range(3))
+        dst = {"new": ht, "gate": gt, "up": ut}[into]
+        n0 = ctx.status().glu_fused
+        ctx.Int4Linear(gt, x, g, rows, hidden, inter)
+        ctx.Int4Linear(ut, x, u, rows, hidden, inter)
+        ctx.Kernel(hip.GO_SWIGLU, rows * inter, dst, gt, ut, None, [inter, 0])
+        assert ctx.status().glu_fused - n0 == int(fuse)
+        got[fuse] = [ctx.Download(t).view(np.uint32).copy() for t in (gt, ut, dst)]
+        for t in (gt, ut, ht):
+            ctx.Recycle(t)
+    for a, b in zip(got["1"], got["0"]):
+        assert np.array_equal(a, b)
+    ctx.Recycle(x)
