@@ -178,8 +178,8 @@ void reload_tuning() {
   t.i4_target_waves = env_int("QNN_I4_TARGET_WAVES", t.i4_target_waves);
   t.i4_sps = env_int("QNN_I4_SPS", t.i4_sps);
   t.i4_wide = env_int("QNN_I4_WIDE", t.i4_wide);
-  t.moe_mt = env_int("QNN_MOE_MT", t.moe_mt);
   t.moe_sps = env_int("QNN_MOE_SPS", t.moe_sps);
+  t.moe_gemm_rows = env_int("QNN_MOE_GEMM_ROWS", t.moe_gemm_rows);
   g_tuning = t;
 }
 
@@ -2466,7 +2466,11 @@ int qnn_moe_experts(qnn_ctx *ctx, qnn_expert_set *set, qnn_tensor *dst, qnn_tens
     const MoEPlanSizes p = moe_plan(a);
     const size_t n = size_t(rows) * topk;
     const size_t hfl = (n * set->inter + 63) / 64 * 64;
-    float *w = static_cast<float *>(ensure_work(ctx, (hfl + n * set->hidden) * 4));
+    const size_t hy = (hfl + (n * set->hidden + 63) / 64 * 64) * 4;
+    const bool gemm = moe_gemm_applies(a);
+    MoEGemm mm;
+    float *w = static_cast<float *>(ensure_work(ctx, hy + (gemm ? moe_gemm_bytes(a, mm, nullptr) : 0)));
+    if (gemm) moe_gemm_bytes(a, mm, reinterpret_cast<uint8_t *>(w) + hy);
     a.h = w;
     a.y = w + hfl;
     ensure_splitk(ctx, p.partial_floats + p.plan_words, p.counters);
@@ -2514,7 +2518,8 @@ int qnn_moe_experts(qnn_ctx *ctx, qnn_expert_set *set, qnn_tensor *dst, qnn_tens
       fr.on = false;
       misc_moe_route(fr.routes, fr.logits, 1, fr.experts, fr.k, fr.normalize, ctx->stream);
     }
-    moe_launch(a, p, ctx->stream);
+    if (gemm) moe_gemm_launch(a, mm, p, ctx->stream);
+    else moe_launch(a, p, ctx->stream);
     return QNN_OK;
   });
 }

@@ -572,6 +572,58 @@ __device__ __forceinline__ void mf_to_rows(float (&acc)[MT], const float (&accm)
   for (int m = 0; m < MT; ++m) acc[m] = slot[m * 64 + lane];
 }
 
+// ---- Weights as exact fp16 integers, for the fp16 matrix cores (many rows:
+// qnn_int4_gemm.hip, the multi-token experts of qnn_moe.hip).
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ half2v as_half2(uint32_t v) {
+  half2v h;
+  __builtin_memcpy(&h, &v, 4);
+  return h;
+}
+// q - 8 of a packed dword's 8 nibbles, in the order 0 4 1 5 2 6 3 7.  The
+// masks come in registers (i4_masks): as literals the and and the or would
+// not fit one v_and_or_b32.
+struct I4Masks {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ I4Masks i4_masks() {
+  I4Masks m;
+  asm("v_mov_b32 %0, 0xf000f" : "=v"(m.lo));
+  asm("v_mov_b32 %0, 0xf000f0" : "=v"(m.hi));
+  return m;
+}
+__device__ __forceinline__ half8 unpack_i4(uint32_t w, const I4Masks &mk) {
+  const uint32_t lo = mk.lo, hi = mk.hi, ex = 0x64006400u, w8 = w >> 8;  // 0x6400: 1024 in fp16
+  const half2v off = {_Float16(-1032.0f), _Float16(-1032.0f)};                        // 1024 + q
+  const half2v six = {_Float16(0.0625f), _Float16(0.0625f)}, off16 = {_Float16(-72.0f), _Float16(-72.0f)};  // 1024 + 16 q
+  half2v v[4];
+  v[0] = as_half2((w & lo) | ex) + off;
+  v[1] = __builtin_elementwise_fma(as_half2((w & hi) | ex), six, off16);
+  v[2] = as_half2((w8 & lo) | ex) + off;
+  v[3] = __builtin_elementwise_fma(as_half2((w8 & hi) | ex), six, off16);
+  half8 r;
+  __builtin_memcpy(&r, v, 16);
+  return r;
+}
+
+// An activation row's planes: v = x 2^-e (exact), hi = fp16(v), lo = fp16(v -
+// hi); an infinity or NaN is in hi alone.  act_exp: the row's e from its
+// largest magnitude; below 2^-110 rows keep that scale, which stays finite.
+__device__ __forceinline__ int act_exp(float amax) { return max(range_exp(amax), -110); }
+// 8 elements -> two pieces of 8 halfs in unpack_i4's order.
+__device__ __forceinline__ void act_planes(const float (&x)[8], float scale, uint4 &ph, uint4 &pl) {
+  float hi[8], lo[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float s = x[i] * scale;
+    hi[i] = float(_Float16(s));
+    lo[i] = isfinite(hi[i]) ? s - hi[i] : 0.0f;
+  }
+  ph = make_uint4(pack_h2(hi[0], hi[4]), pack_h2(hi[1], hi[5]), pack_h2(hi[2], hi[6]), pack_h2(hi[3], hi[7]));
+  pl = make_uint4(pack_h2(lo[0], lo[4]), pack_h2(lo[1], lo[5]), pack_h2(lo[2], lo[6]), pack_h2(lo[3], lo[7]));
+}
+
 // Sum over the L lanes of each row (L a power of two): afterwards every lane
 // of a row holds the row total.  Pairwise order, identical in every launch.
 template <int MT>

@@ -57,9 +57,9 @@
 namespace qnn {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+using dev::half8;
+using dev::I4Masks;
 using dev::Rsrc;
 
 // ---- activations ------------------------------------------------------------
@@ -109,22 +109,13 @@ __global__ __launch_bounds__(1024) void k_i4_act(const float *__restrict__ x, in
   amax = dev::wave_max_xor(amax);
   if (lane == 0) red[rw][part] = amax;
   __syncthreads();
-  // Rows below 2^-110 keep that scale, which stays finite.
-  const int e = max(range_exp(fmaxf(fmaxf(red[rw][0], red[rw][1]), fmaxf(red[rw][2], red[rw][3]))), -110);
+  const int e = dev::act_exp(fmaxf(fmaxf(red[rw][0], red[rw][1]), fmaxf(red[rw][2], red[rw][3])));
   if (t == 0 && blockIdx.y == 0) ex[row] = e;
   const float sc = ldexpf(1.0f, -e);
   auto put = [&](int c, const float (&v)[8]) {
-    float hi[8], lo[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float s = v[i] * sc;  // exact: a power of two
-      hi[i] = float(_Float16(s));
-      lo[i] = isfinite(hi[i]) ? s - hi[i] : 0.0f;  // an infinity or NaN is in hi alone
-    }
     const int g = c >> 2, d = c & 3;
     uint4 *dst = frag + ((size_t(row >> 5) * gpad + g) * 4 + (d & 1)) * 64 + (row & 31) + 32 * (d >> 1);
-    dst[0] = make_uint4(pack_h2(hi[0], hi[4]), pack_h2(hi[1], hi[5]), pack_h2(hi[2], hi[6]), pack_h2(hi[3], hi[7]));
-    dst[128] = make_uint4(pack_h2(lo[0], lo[4]), pack_h2(lo[1], lo[5]), pack_h2(lo[2], lo[6]), pack_h2(lo[3], lo[7]));
+    dev::act_planes(v, sc, dst[0], dst[128]);
   };
   if (c0 < c1) put(c0, first);
   for (int c = c0 + 256; c < c1; c += 256) {
@@ -144,37 +135,6 @@ struct I4GemmArgs {
   float *part;                // K-split: partial sums [slice][matrix][M][N]
   int M, N, gpad, m32, tiles, slices, ktiles;
 };
-
-__device__ __forceinline__ half2v as_half2(uint32_t v) {
-  half2v h;
-  __builtin_memcpy(&h, &v, 4);
-  return h;
-}
-// q - 8 of a packed dword's 8 nibbles, in the order 0 4 1 5 2 6 3 7.  The
-// masks come in registers (i4_masks): as literals the and and the or would
-// not fit one v_and_or_b32.
-struct I4Masks {
-  uint32_t lo, hi;
-};
-__device__ __forceinline__ I4Masks i4_masks() {
-  I4Masks m;
-  asm("v_mov_b32 %0, 0xf000f" : "=v"(m.lo));
-  asm("v_mov_b32 %0, 0xf000f0" : "=v"(m.hi));
-  return m;
-}
-__device__ __forceinline__ half8 unpack_i4(uint32_t w, const I4Masks &mk) {
-  const uint32_t lo = mk.lo, hi = mk.hi, ex = 0x64006400u, w8 = w >> 8;  // 0x6400: 1024 in fp16
-  const half2v off = {_Float16(-1032.0f), _Float16(-1032.0f)};                        // 1024 + q
-  const half2v six = {_Float16(0.0625f), _Float16(0.0625f)}, off16 = {_Float16(-72.0f), _Float16(-72.0f)};  // 1024 + 16 q
-  half2v v[4];
-  v[0] = as_half2((w & lo) | ex) + off;
-  v[1] = __builtin_elementwise_fma(as_half2((w & hi) | ex), six, off16);
-  v[2] = as_half2((w8 & lo) | ex) + off;
-  v[3] = __builtin_elementwise_fma(as_half2((w8 & hi) | ex), six, off16);
-  half8 r;
-  __builtin_memcpy(&r, v, 16);
-  return r;
-}
 
 // 16 bytes per lane from global memory into LDS at `lds` (uniform).
 // The compiler does not see the write: gemm_vmwait and the barriers order it.
@@ -258,7 +218,7 @@ __global__ __launch_bounds__(512) void k_i4_gemm(const I4GemmArgs a) {
 #pragma unroll
     for (int i = 0; i < SG::LPW; ++i) load_one(k, i);
 
-  const I4Masks masks = i4_masks();
+  const I4Masks masks = dev::i4_masks();
   float acc[MB][2][16];
   f32x16 d[2][2];
 #pragma unroll
@@ -292,8 +252,8 @@ __global__ __launch_bounds__(512) void k_i4_gemm(const I4GemmArgs a) {
   // Row l's dwords (lane l) -> dword 2h + kk of row 32 t + lane % 32 (h = lane / 32).
   auto unpack_pair = [&](half8 (&f)[2][2], uint32_t d0, uint32_t d2, int kk) {
     const auto r = __builtin_amdgcn_permlane32_swap(d0, d2, false, false);
-    f[0][kk] = unpack_i4(r[0], masks);
-    f[1][kk] = unpack_i4(r[1], masks);
+    f[0][kk] = dev::unpack_i4(r[0], masks);
+    f[1][kk] = dev::unpack_i4(r[1], masks);
   };
 
   // One K-tile (P: its parity).  Phase i runs the 8 MFMAs of row block i, two

@@ -58,8 +58,8 @@ struct Tuning {
   int i4_target_waves = 0;   // QNN_I4_TARGET_WAVES: wave target of the INT4 planner
   int i4_sps = 0;            // QNN_I4_SPS: INT4 steps per wave
   int i4_wide = 1;           // QNN_I4_WIDE: one-token 8/16-wave workgroups
-  int moe_mt = 0;            // QNN_MOE_MT: tokens per pass of the multi-token MoE kernels
   int moe_sps = 0;           // QNN_MOE_SPS: MoE steps per wave
+  int moe_gemm_rows = 2;     // QNN_MOE_GEMM_ROWS: rows from which routed experts run on the matrix cores (0: never)
 };
 const Tuning &tuning();
 void reload_tuning();
@@ -311,6 +311,14 @@ struct MoELaunch {
   float *routes_out = nullptr;    // the route tensor, written as GO_MOE_ROUTE would
   int normalize = 0;
 };
+// The matrix-core launches of several tokens: the token rows' and the h rows'
+// fp16 planes, [row][gpad groups][2][4] pieces of 16 bytes, and their
+// exponents (set by moe_gemm_bytes).
+struct MoEGemm {
+  uint4 *xfrag = nullptr, *hfrag = nullptr;
+  int *xexp = nullptr, *hexp = nullptr;
+  int gpad_x = 0, gpad_h = 0;
+};
 struct MoEPlanSizes {
   int slots = 0, mt = 1, gsw = 4, slices_gu = 1, slices_dn = 1, sps_gu = 1, sps_dn = 1;
   size_t lds_gu = 0, lds_dn = 0;  // dynamic LDS per launch
@@ -329,6 +337,11 @@ int moe_decode_capacity(const MoEPlanSizes &p, int route_j, int device);  // co-
 bool moe_decode_launch(const MoELaunch &a, const MoEPlanSizes &p, const MoEDecodePlan &d, int route_j, hipStream_t s);
 MoEPlanSizes moe_plan(const MoELaunch &a);
 void moe_launch(const MoELaunch &a, const MoEPlanSizes &p, hipStream_t s);
+// Several tokens on the matrix cores: whether the rule takes them; the
+// workspace, whose pointers it sets in `g` for a workspace at `ws`; the launches.
+bool moe_gemm_applies(const MoELaunch &a);
+size_t moe_gemm_bytes(const MoELaunch &a, MoEGemm &g, uint8_t *ws);
+void moe_gemm_launch(const MoELaunch &a, const MoEGemm &g, const MoEPlanSizes &p, hipStream_t s);
 
 // Multi-row Q8_0 projection on fp16 MFMA (qnn_gemm.hip).
 struct Q8GemmPlan {

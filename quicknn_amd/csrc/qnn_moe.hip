@@ -21,7 +21,8 @@
 // per launch for all of its tokens.  Split-K slices of a
 // (slot, tile) are combined by the last to finish, and in the down launch the
 // last (slot, tile) of a tile to finish combines the experts, both in a fixed
-// order, so results do not depend on timing.
+// order, so results do not depend on timing.  Several tokens take the matrix
+// cores instead (k_moe_mm); one token has a launch of its own (k_moe_decode).
 #include "qnn_int4_dev.h"
 #include "qnn_route_dev.h"
 
@@ -119,6 +120,49 @@ __device__ void build_order(MoEPlan &pl, int n, int k, int lane) {
   }
 }
 
+// One wave: a row's two fp16 planes (dev::act_planes) and its exponent, in
+// row-major pieces [row][group][plane][dword] of 16 bytes.
+constexpr int kActHold = 4;
+__device__ void act_row(const float *__restrict__ x, int row, int K, int gpad, int *__restrict__ ex,
+                        uint4 *__restrict__ frag, int lane) {
+  const float *r = x + size_t(row) * K;
+  const int chunks = 4 * gpad;
+  auto load8 = [&](int c, float (&v)[8]) {  // K % 4 == 0, 16-byte aligned rows
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+    if (8 * c < K) a = *reinterpret_cast<const float4 *>(r + 8 * c);
+    if (8 * c + 4 < K) b = *reinterpret_cast<const float4 *>(r + 8 * c + 4);
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+  };
+  float held[kActHold][8], amax = 0.0f;
+#pragma unroll
+  for (int h = 0; h < kActHold; ++h) load8(lane + 64 * h, held[h]);
+#pragma unroll
+  for (int h = 0; h < kActHold; ++h)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(held[h][i]));
+  for (int c = lane + 64 * kActHold; c < chunks; c += 64) {
+    float v[8];
+    load8(c, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+  }
+  const int e = dev::act_exp(dev::wave_max_xor(amax));
+  if (lane == 0) ex[row] = e;
+  const float sc = ldexpf(1.0f, -e);
+  auto put = [&](int c, const float (&v)[8]) {
+    uint4 *dst = frag + (size_t(row) * gpad + (c >> 2)) * 8 + (c & 3);
+    dev::act_planes(v, sc, dst[0], dst[4]);
+  };
+#pragma unroll
+  for (int h = 0; h < kActHold; ++h)
+    if (lane + 64 * h < chunks) put(lane + 64 * h, held[h]);
+  for (int c = lane + 64 * kActHold; c < chunks; c += 64) {
+    float v[8];
+    load8(c, v);
+    put(c, v);
+  }
+}
+
 // Multi-token launches: every slot's plan is built once per call by
 // k_moe_plan (the same build_plan / build_order that each workgroup ran
 // itself before) and stored as a record per slot -- expert, position count,
@@ -127,12 +171,16 @@ __device__ void build_order(MoEPlan &pl, int n, int k, int lane) {
 // loads instead of rebuilding the plan (batch 16: building it twice per
 // workgroup cost 16 us per layer).
 constexpr int kSlotWords = 4 + kMaxPos;
-// Workgroups 0 .. slots-1 build one slot's record each; the last one (slot
+// Workgroups 0 .. slots-1 build one slot's record each; the next one (slot
 // == slots) writes the route ids and the per-token order, in parallel with
-// them.
-__global__ __launch_bounds__(64) void k_moe_plan(const MoELaunch a, const int slots) {
+// them; for the matrix-core launches the rest prepare one token row each.
+__global__ __launch_bounds__(64) void k_moe_plan(const MoELaunch a, const MoEGemm mm, const int slots) {
   __shared__ MoEPlan pl;
   const int n = a.rows * a.topk, slot = blockIdx.x, lane = threadIdx.x;
+  if (slot > slots) {
+    act_row(a.x, slot - slots - 1, a.hidden, mm.gpad_x, mm.xexp, mm.xfrag, lane);
+    return;
+  }
   if (slot == slots) {
     for (int i = lane; i < n; i += 64) pl.ids[i] = __float_as_uint(a.routes[i]);
     dev::wave_lds_sync();
@@ -410,12 +458,227 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
   if (wave == 0) dev::reset_counter(&a.counters[(size_t(tiles) * slots + tile) * kCounterStride], lane);
 }
 
+// ---- several tokens on the fp16 matrix cores ----------------------------------
+// An expert's tokens (a prompt chunk of 128 tokens, top 8 of 128 experts: 8 on
+// average) as one small product per 64-row weight block: the arithmetic of
+// qnn_int4_gemm.hip (activations as two fp16 planes per row, exact fp16
+// weights, each group's sum from zero, folded with its fp32 scale) on 16 x 16
+// tiles, v_mfma_f32_16x16x32_f16 taking a whole group of 16 tokens x 16 weight
+// rows.  Every routed weight is unpacked once for up to 16 TT tokens, where
+// k_moe makes a pass of 16 v_dot4 and a staging barrier per token (gate/up
+// 185 us, down 147 us at that chunk).  What bounds it is the weight stream;
+// per 64 x 32 weights the VALU has 56 operations.
+// * the planning launch prepares the token rows too, k_moe_act the h rows
+//   between the launches.  Pieces are row-major, so a lane gathers its token's
+//   piece from wherever the row is.
+// * gate/up (k_moe_mm<.., false>): a workgroup is one block of one slot, its
+//   eight waves the gate and the up matrix in four K-quarters each, which meet
+//   in LDS: no exchange between workgroups.
+// * down (<.., true>): a workgroup is four blocks, two waves (K-halves) each.
+// * k_moe_combine adds a token's experts in ascending id, as k_moe does.
+// The next chunk's weights (four groups) are requested before the current
+// chunk's products; more comes from the four waves per SIMD (a wave's scales
+// go through LDS: as four loads per lane they took 128 registers and spilled).
+//
+// Measured, whole layer with router and route, 128 experts of 768 x 2048, top
+// 8: 128 tokens 525 -> 129 us (338 with the router's share gone; gate/up 69
+// us, 3.6 TB/s, down 43 us), 32 tokens 309 -> 105, 8 tokens 183 -> 66, 2
+// tokens 141 -> 41 us; 8 experts of 256 x 512, top 2, 2 tokens 43 -> 32 us:
+// faster from two tokens on at every shape measured, so from two.
+__global__ __launch_bounds__(256) void k_moe_act(const float *__restrict__ x, int rows, int K, int gpad,
+                                                 int *__restrict__ ex, uint4 *__restrict__ frag) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row < rows) act_row(x, row, K, gpad, ex, frag, threadIdx.x & 63);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+struct MmWeights {  // four groups of a 64-row block
+  uint4 w[4];       // row l's nibbles per group
+  uint4 q;          // row l's four scales
+};
+
+template <int TT, bool DOWN>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TT == 1 ? 4 : 2))) void k_moe_mm(const MoELaunch a, const MoEGemm mm, const int items) {
+  __shared__ float red[8][TT * 16][64];
+  __shared__ uint4 scl[8][64];  // a wave's scales of the chunk: every lane needs four other rows'
+  const int slot = blockIdx.x / items, item = blockIdx.x - slot * items;
+  const int lane = threadIdx.x & 63, wave = dev::wave_id();
+  const int *rec = a.plan + size_t(slot) * kSlotWords;
+  const int e = rec[0], c = rec[1];
+  if (e < 0) return;  // fewer routed experts than slots
+  const I4Layout &l = DOWN ? a.dn : a.gu;
+  const int gpad = DOWN ? mm.gpad_h : mm.gpad_x, chunks = (l.steps + 3) / 4;
+  // Wave: K-part kq of KQ of block b of matrix mat.
+  constexpr int KQ = DOWN ? 2 : 4;
+  const int mat = DOWN ? 0 : wave & 1, kq = DOWN ? wave & 1 : wave >> 1;
+  const int bw_ = DOWN ? item * 4 + (wave >> 1) : item, b = min(bw_, l.blocks - 1);  // past the last: not written
+  const int ch0 = kq * chunks / KQ, ch1 = (kq + 1) * chunks / KQ;
+  const uint8_t *wb = DOWN ? a.down + size_t(e) * a.dn_stride : a.gate_up + size_t(2 * e + mat) * a.gu_stride;
+  // One block's weights: steps past the last read zeros (scale pieces hold zeros there).
+  const dev::Rsrc nr = dev::rsrc(wb + size_t(b) * l.steps * 1024, size_t(l.steps) * 1024);
+  const dev::Rsrc sr = dev::rsrc(wb + l.nib_bytes() + size_t(b) * l.quads() * 1024, size_t(l.quads()) * 1024);
+  const dev::Rsrc xr = DOWN ? dev::rsrc(mm.hfrag, size_t(a.rows) * a.topk * gpad * 128)
+                            : dev::rsrc(mm.xfrag, size_t(a.rows) * gpad * 128);
+  const int p = lane & 15, d = lane >> 4;
+  auto load_w = [&](MmWeights &m, int ch) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      m.w[g] = dev::ld128<dev::kStream>(nr, uint32_t(lane) * 16u, uint32_t(ch * 4 + g) * 1024u);
+    m.q = dev::ld128<dev::kStream>(sr, uint32_t(lane) * 16u, uint32_t(ch) * 1024u);
+  };
+  const dev::I4Masks masks = dev::i4_masks();
+  for (int m0 = 0; m0 < c; m0 += 16 * TT) {
+    uint32_t xoff[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      const int R = rec[4 + min(m0 + 16 * t + p, c - 1)];
+      xoff[t] = uint32_t(DOWN ? R : R / a.topk) * uint32_t(gpad) * 128u + uint32_t(d) * 16u;
+    }
+    f32x4 acc[TT][4];
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](const MmWeights &m, int ch) {
+      uint4 xa[2][TT][2];  // this group's and the next one's token pieces
+      auto load_a = [&](int g) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int pl = 0; pl < 2; ++pl)
+            xa[g & 1][t][pl] = dev::ld128(xr, xoff[t], uint32_t(ch * 4 + g) * 128u + uint32_t(pl) * 64u);
+      };
+      load_a(0);
+      dev::wave_lds_sync();  // the previous chunk's scales are read
+      scl[wave][lane] = m.q;
+      dev::wave_lds_sync();
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (g < 3) load_a(g + 1);
+        float sc[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[r] = reinterpret_cast<const float *>(&scl[wave][16 * r + p])[g];
+        uint32_t wq[4];
+        dev::mf_transpose(wq, m.w[g]);  // dword d of row 16 r + p
+        dev::half8 bw[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bw[r] = dev::unpack_i4(wq[r], masks);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          dev::half8 xh, xl;
+          __builtin_memcpy(&xh, &xa[g & 1][t][0], 16);
+          __builtin_memcpy(&xl, &xa[g & 1][t][1], 16);
+          f32x4 s[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            s[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, bw[r], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, bw[r], s[r], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[t][r][i] = fmaf(s[r][i], sc[r], acc[t][r][i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one group's unpacked weights at a time
+      }
+    };
+    MmWeights w0, w1;
+    int ch = ch0;
+    if (ch < ch1) load_w(w0, ch);
+    for (; ch + 1 < ch1; ch += 2) {
+      load_w(w1, ch + 1);
+      products(w0, ch);
+      load_w(w0, min(ch + 2, ch1 - 1));
+      products(w1, ch + 1);
+    }
+    if (ch < ch1) products(w0, ch);
+
+    // Lane: weight row 16 r + p, tokens 4 d + i of tile t.
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[wave][(t * 4 + r) * 4 + i][lane] = acc[t][r][i];
+    __syncthreads();
+    // Gate/up: wave w finishes outputs w, w + 8, ..; down: its block's w % 2, ...
+#pragma unroll
+    for (int j = 0; j < (DOWN ? 8 : 2) * TT; ++j) {
+      const int o = DOWN ? (wave & 1) + 2 * j : wave + 8 * j, t = o >> 4, r = (o >> 2) & 3, i = o & 3;
+      const int m = m0 + 16 * t + 4 * d + i, n = bw_ * 64 + 16 * r + p;
+      if (m >= c || n >= (DOWN ? a.hidden : a.inter)) continue;
+      const int R = rec[4 + m];
+      if constexpr (DOWN) {
+        a.y[size_t(R) * a.hidden + n] = ldexpf(red[wave & ~1][o][lane] + red[wave | 1][o][lane], mm.hexp[R]);
+      } else {
+        const int x = mm.xexp[R / a.topk];
+        float g = 0.0f, u = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          g += red[2 * k][o][lane];
+          u += red[2 * k + 1][o][lane];
+        }
+        a.h[size_t(R) * a.inter + n] = dev::silu(ldexpf(g, x)) * ldexpf(u, x);
+      }
+    }
+    __syncthreads();  // red is rewritten by the next tokens
+  }
+}
+
+// out[t] = sum over the token's routes in ascending expert id of p * y
+// (moe.comp:70 / :126), four columns per thread.
+__global__ __launch_bounds__(256) void k_moe_combine(const MoELaunch a, const int slots) {
+  const int t = blockIdx.y, j = (blockIdx.x * 256 + threadIdx.x) * 4, n = a.rows * a.topk;
+  if (j >= a.hidden) return;
+  const int *ids = a.plan + size_t(slots) * kSlotWords;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  constexpr int CR = 8;  // routes in flight
+  for (int r0 = 0; r0 < a.topk; r0 += CR) {
+    float4 v[CR];
+    float pv[CR];
+    bool ok[CR];
+#pragma unroll
+    for (int u = 0; u < CR; ++u) {
+      const int R = t * a.topk + ids[n + t * a.topk + min(r0 + u, a.topk - 1)];
+      ok[u] = r0 + u < a.topk && uint32_t(ids[R]) < uint32_t(a.experts);
+      pv[u] = a.routes[n + R];
+      v[u] = *reinterpret_cast<const float4 *>(a.y + size_t(R) * a.hidden + j);
+    }
+#pragma unroll
+    for (int u = 0; u < CR; ++u)
+      if (ok[u]) {
+        acc.x = add_mul_nofma(acc.x, v[u].x, pv[u]);
+        acc.y = add_mul_nofma(acc.y, v[u].y, pv[u]);
+        acc.z = add_mul_nofma(acc.z, v[u].z, pv[u]);
+        acc.w = add_mul_nofma(acc.w, v[u].w, pv[u]);
+      }
+  }
+  *reinterpret_cast<float4 *>(a.out + size_t(t) * a.hidden + j) = acc;
+}
+
+void launch_mm(const MoELaunch &a, const MoEGemm &mm, const MoEPlanSizes &p, hipStream_t s) {
+  const int n = a.rows * a.topk, idn = (a.dn.blocks + 3) / 4;
+  hipLaunchKernelGGL(k_moe_plan, dim3(p.slots + 1 + a.rows), dim3(64), 0, s, a, mm, p.slots);
+  // Two tiles of 16 tokens where an expert has more than 16 as a rule.
+  if (n > 24 * a.experts) {
+    hipLaunchKernelGGL((k_moe_mm<2, false>), dim3(p.slots * a.gu.blocks), dim3(512), 0, s, a, mm, a.gu.blocks);
+    hipLaunchKernelGGL(k_moe_act, dim3((n + 3) / 4), dim3(256), 0, s, a.h, n, a.inter, mm.gpad_h, mm.hexp, mm.hfrag);
+    hipLaunchKernelGGL((k_moe_mm<2, true>), dim3(p.slots * idn), dim3(512), 0, s, a, mm, idn);
+  } else {
+    hipLaunchKernelGGL((k_moe_mm<1, false>), dim3(p.slots * a.gu.blocks), dim3(512), 0, s, a, mm, a.gu.blocks);
+    hipLaunchKernelGGL(k_moe_act, dim3((n + 3) / 4), dim3(256), 0, s, a.h, n, a.inter, mm.gpad_h, mm.hexp, mm.hfrag);
+    hipLaunchKernelGGL((k_moe_mm<1, true>), dim3(p.slots * idn), dim3(512), 0, s, a, mm, idn);
+  }
+  hipLaunchKernelGGL(k_moe_combine, dim3((a.hidden / 4 + 255) / 256, a.rows), dim3(256), 0, s, a, p.slots);
+  hip_check(hipGetLastError(), "moe launch");
+}
+
 template <int MT, int GSW>
 void launch_mt(const MoELaunch &a, const MoEPlanSizes &p, hipStream_t s) {
   const int tgu = 2 * a.gu.blocks, tdn = a.dn.blocks;
   const int ggu = (tgu + 7) / 8 * 8 * p.slots * p.slices_gu;
   const int gdn = (tdn + 7) / 8 * 8 * p.slots * p.slices_dn;
-  hipLaunchKernelGGL(k_moe_plan, dim3(p.slots + 1), dim3(64), 0, s, a, p.slots);
+  hipLaunchKernelGGL(k_moe_plan, dim3(p.slots + 1), dim3(64), 0, s, a, MoEGemm(), p.slots);
   hipLaunchKernelGGL((k_moe<MT, GSW, false>), dim3(ggu), dim3(256), p.lds_gu, s, a, p.slices_gu, p.sps_gu, p.slots);
   hipLaunchKernelGGL((k_moe<MT, GSW, true>), dim3(gdn), dim3(256), p.lds_dn, s, a, p.slices_dn, p.sps_dn, p.slots);
 }
@@ -715,28 +978,19 @@ MoEPlanSizes moe_plan(const MoELaunch &a) {
   MoEPlanSizes p;
   const int n = a.rows * a.topk;
   p.slots = std::min(a.experts, n);
-  // One token per pass: fewer registers (at 4 steps per wave 97-114 VGPRs
-  // against 123-126 at 2 tokens); measured faster at 4, 16 and 32 tokens (16:
-  // 159 against 167 us, 100.7 against 123.2 us with the current kernels) even
-  // though an expert with several tokens makes several passes over its
-  // weights in registers.  QNN_MOE_MT (1, 2, 4) overrides.
+  // One token per pass (one token in all, unless the matrix-core launches are
+  // turned off).
   p.mt = 1;
-  const int fmt = tuning().moe_mt;
-  if (fmt == 1 || fmt == 2 || fmt == 4) p.mt = fmt;
-  // Steps per wave: 8 with one token per pass, 4 with several, measured
-  // fastest for 128 experts of 768 x 2048 (one token per pass, 2-64 rows: 8
-  // steps 4-17% faster than 4, e.g. 16 rows 129 -> 114 us, 100.7 against
-  // 118.3 us with the current kernels; 2 tokens per pass: 4 steps 14-16%
-  // faster than 2 and than 8).  One row with its routes given would take 4
-  // (13.36 against 13.63 us), but the launch that computes the routes itself
-  // is faster at 8 (16.55 against 17.91 us) and must sum in the same order as
-  // the routes-given launch, so one row keeps 8.  QNN_MOE_SPS overrides.
+  // Steps per wave: 8.  One row with its routes given would take 4 (13.36
+  // against 13.63 us), but the launch that computes the routes itself is
+  // faster at 8 (16.55 against 17.91 us) and must sum in the same order as the
+  // routes-given launch, so one row keeps 8.  QNN_MOE_SPS overrides.
   // Bounded by the activation-slice LDS budget.
   const int forced = tuning().moe_sps;
   auto steps = [&](const I4Layout &l, int) {
     const int lds_cap = int((48 << 10) / (size_t(p.mt) * 4 * l.lanes * (dev::kXWords * 4 + 8)));
     const int cap = std::max(1, std::min(8, lds_cap));
-    return std::min(forced > 0 ? forced : (p.mt == 1 ? 8 : 4), cap);
+    return std::min(forced > 0 ? forced : 8, cap);
   };
   p.sps_gu = steps(a.gu, 2 * a.gu.blocks);
   p.sps_dn = steps(a.dn, a.dn.blocks);
@@ -753,20 +1007,39 @@ MoEPlanSizes moe_plan(const MoELaunch &a) {
   return p;
 }
 
+size_t moe_gemm_bytes(const MoELaunch &a, MoEGemm &mm, uint8_t *ws) {
+  const size_t n = size_t(a.rows) * a.topk;
+  mm.gpad_x = (a.gu.groups + 3) / 4 * 4;
+  mm.gpad_h = (a.dn.groups + 3) / 4 * 4;
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    uint8_t *p = ws + at;
+    at += (bytes + 255) / 256 * 256;
+    return p;
+  };
+  mm.xfrag = reinterpret_cast<uint4 *>(take(size_t(a.rows) * mm.gpad_x * 128));
+  mm.hfrag = reinterpret_cast<uint4 *>(take(n * mm.gpad_h * 128));
+  mm.xexp = reinterpret_cast<int *>(take(size_t(a.rows) * 4));
+  mm.hexp = reinterpret_cast<int *>(take(n * 4));
+  return at;
+}
+
+void moe_gemm_launch(const MoELaunch &a, const MoEGemm &mm, const MoEPlanSizes &p, hipStream_t s) {
+  launch_mm(a, mm, p, s);
+}
+
+bool moe_gemm_applies(const MoELaunch &a) {
+  const int from = tuning().moe_gemm_rows;
+  return from > 0 && a.rows >= from && size_t(a.rows) * a.topk * ((a.dn.groups + 3) / 4 * 4) * 128 <= 0xFFFFFFFFull &&
+         size_t(a.rows) * ((a.gu.groups + 3) / 4 * 4) * 128 <= 0xFFFFFFFFull;
+}
+
 void moe_launch(const MoELaunch &a, const MoEPlanSizes &p, hipStream_t s) {
   switch (p.mt * 16 + p.gsw) {
     case 1 * 16 + 1: launch_mt<1, 1>(a, p, s); break;
     case 1 * 16 + 2: launch_mt<1, 2>(a, p, s); break;
     case 1 * 16 + 4: launch_mt<1, 4>(a, p, s); break;
     case 1 * 16 + 8: launch_mt<1, 8>(a, p, s); break;
-    case 2 * 16 + 1: launch_mt<2, 1>(a, p, s); break;
-    case 2 * 16 + 2: launch_mt<2, 2>(a, p, s); break;
-    case 2 * 16 + 4: launch_mt<2, 4>(a, p, s); break;
-    case 2 * 16 + 8: launch_mt<2, 8>(a, p, s); break;
-    case 4 * 16 + 1: launch_mt<4, 1>(a, p, s); break;
-    case 4 * 16 + 2: launch_mt<4, 2>(a, p, s); break;
-    case 4 * 16 + 4: launch_mt<4, 4>(a, p, s); break;
-    case 4 * 16 + 8: launch_mt<4, 8>(a, p, s); break;
     default: fail(QNN_E_INVALID_OP, "MoE launch plan");
   }
   hip_check(hipGetLastError(), "moe launch");

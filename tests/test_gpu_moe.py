@@ -398,3 +398,36 @@ def test_route_over_1024_experts_is_not_recorded(ctx, rng):
     assert np.array_equal(got[:k].view(np.uint32), ids[0])
     ctx.Recycle(lt)
     ctx.Recycle(rt)
+
+
+@pytest.mark.parametrize("E,hidden,inter,k,rows", [
+    (4, 64, 64, 1, 2),       # whole groups, one block
+    (5, 36, 40, 2, 3),       # partial groups, partial blocks
+    (2, 132, 68, 2, 17),     # an expert with 17 tokens: a second pass of 16
+    (3, 2080, 324, 2, 33),   # more activation pieces than a wave holds, five blocks of h, 65 groups in K-quarters
+    (1, 128, 260, 1, 128),   # every token, two tiles of 16 per pass
+    (2, 68, 132, 1, 70),     # two tiles, ragged
+    (300, 96, 96, 7, 60),    # most experts with one token
+])
+def test_moe_experts_matrix_core_launches(ctx, rng, tune, E, hidden, inter, k, rows):
+    """Several tokens on the matrix cores against the one-token path's kernels (QNN_MOE_GEMM_ROWS=0), which hold
+    activations in 16 bits per group (2e-5 each way), and the CPU path; twice the same bits."""
+    ex = Experts(rng, E, hidden, inter)
+    s = ctx.CreateExpertSet(ex.bg, ex.bu, ex.bd, hidden, inter)
+    x = rng.standard_normal((rows, hidden)).astype(np.float32)
+    routes, ids, probs = route_on_gpu(ctx, rng.standard_normal((rows, E)).astype(np.float32), k)
+    src = ctx.UploadRaw(x)
+    got = {}
+    for name, frm in (("mm", "2"), ("again", "2"), ("dot", "0")):
+        tune("QNN_MOE_GEMM_ROWS", frm)
+        dst = ctx.UploadRaw(np.full(rows * hidden + 32, 7.0, np.float32))
+        ctx.MoEExperts(s, dst, src, routes, rows, k)
+        got[name] = ctx.Download(dst)
+        assert np.all(got[name][rows * hidden:] == 7.0)
+    ctx.DestroyExpertSet(s)
+    assert np.array_equal(got["mm"].view(np.uint32), got["again"].view(np.uint32))
+    mm, dot = (got[n][:rows * hidden].reshape(rows, hidden) for n in ("mm", "dot"))
+    want = ex.oracle(x, ids, probs)
+    for r in range(rows):
+        assert normwise_rel_err(mm[r], dot[r]) <= 2e-4, r
+        assert normwise_rel_err(mm[r], want[r]) <= TOL, r
