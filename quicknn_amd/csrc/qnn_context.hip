@@ -166,6 +166,7 @@ void reload_tuning() {
   t.gemm_max_rows = env_int("QNN_GEMM_MAX_ROWS", t.gemm_max_rows);
   t.attn_wgs = env_int("QNN_ATTN_WGS", t.attn_wgs);
   t.attn_min_chunk = env_int("QNN_ATTN_MIN_CHUNK", t.attn_min_chunk);
+  t.attn_mm_min = env_int("QNN_ATTN_MM", t.attn_mm_min);
   t.attn_dma = env_int("QNN_ATTN_DMA", t.attn_dma);
   t.gemm_nw = env_int("QNN_GEMM_NW", t.gemm_nw);
   t.gemm_mb = env_int("QNN_GEMM_MB", t.gemm_mb);
@@ -2276,7 +2277,7 @@ int qnn_cached_attention(qnn_ctx *ctx, qnn_tensor *dst, qnn_tensor *q, qnn_tenso
     check_tensor(ctx, q, int64_t(query_rows) * heads * dim);
     check_tensor(ctx, dst, int64_t(query_rows) * heads * dim);
     check_tensor(ctx, cache, 2 * int64_t(capacity) * kv_heads * dim + (masked ? int64_t(query_rows) * capacity : 0));
-    const AttnPlan p = attn_plan(query_rows, heads, kv_heads, dim, position, window);
+    const AttnPlan p = attn_plan(query_rows, capacity, heads, kv_heads, dim, position, window);
     float *ws = p.part_floats ? static_cast<float *>(ensure_work(ctx, p.part_floats * 4)) : nullptr;
     attn_launch(q->ptr, cache->ptr, dst->ptr, ws, p, query_rows, capacity, heads, kv_heads, dim, position, window,
                 softcap, scale, masked ? 1 : 0, ctx->stream);

@@ -1190,8 +1190,9 @@ void decode_softcap(float *dst, const float *src, int n, float cap, hipStream_t 
   k_softcap<<<grid_of(n, 256), 256, 0, s>>>(dst, src, n, cap);
 }
 
-AttnPlan attn_plan(int rows, int heads, int kv_heads, int dim, int position, int window) {
+AttnPlan attn_plan(int rows, int cap, int heads, int kv_heads, int dim, int position, int window) {
   AttnPlan p;
+  if (attn_mm_plan(p, rows, cap, heads, kv_heads, dim, position, window)) return p;
   const int group = heads / kv_heads;
   p.gb = group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
   const int wgs = kv_heads * (group / p.gb) * rows;
@@ -1238,9 +1239,12 @@ void attn_launch(const float *q, const float *cache, float *out, float *ws, cons
                                size_t(a.kl > 1 ? a.kl : 0) * p.gb * dim);
   const size_t lds = (size_t(p.gb) * dim + size_t(p.gb) * kAttnSub + p.gb * 4 + xred) * 4;
   dim3 grid(kv_heads * a.gpk, rows, p.splits);
+  const bool mm = p.qtiles > 0;
+  if (mm)
+    attn_mm_launch(q, cache, out, opart, ml, p, rows, cap, heads, kv_heads, dim, position, window, softcap, scale, masked, s);
   // The LDS-stream kernel: dim 128, 64-key chunks, every chunk start a multiple
   // of 4 keys (16-byte K^T pieces), and a capacity of whole 16-byte rows.
-  bool dma = tuning().attn_dma != 0 && dim == kDmaDim && p.chunk == kDmaKeys && cap % 4 == 0 && a.kl == 8 &&
+  bool dma = !mm && tuning().attn_dma != 0 && dim == kDmaDim && p.chunk == kDmaKeys && cap % 4 == 0 && a.kl == 8 &&
              a.lpk == 32 && a.parts == 4;
   for (int r = 0; dma && r < rows; ++r) {
     const int e = position + r + 1;
@@ -1266,7 +1270,7 @@ void attn_launch(const float *q, const float *cache, float *out, float *ws, cons
     }
   }
 #define QNN_ATTN(G, N) k_attn<G, N><<<grid, kAttnThreads, lds, s>>>(q, cache, out, opart, ml, a)
-  if (dma) {
+  if (mm || dma) {
   } else if (a.nd4 == 1) {
     switch (p.gb) {
       case 8: QNN_ATTN(8, 1); break;

@@ -46,6 +46,7 @@ struct Tuning {
   int gemm_max_rows = 0;     // QNN_GEMM_MAX_ROWS: rows per GEMM launch, at most (0: the 4 GiB fragment limit)
   int attn_wgs = 512;        // QNN_ATTN_WGS: cached-attention workgroup target
   int attn_min_chunk = 64;   // QNN_ATTN_MIN_CHUNK: keys per chunk, at least
+  int attn_mm_min = 512;     // QNN_ATTN_MM: rows x heads x keys, in 1024s, from which attention of several rows takes the matrix cores (0: never)
   int attn_dma = 1;          // QNN_ATTN_DMA: 64-key chunks at dim 128 streamed into LDS
   int gemm_nw = 0;           // QNN_GEMM_NW: waves per Q8_0 GEMM workgroup (4 or 8)
   int gemm_mb = 0;           // QNN_GEMM_MB: 32-row blocks per GEMM wave (1 or 2)
@@ -242,9 +243,15 @@ void decode_softcap(float *dst, const float *src, int n, float cap, hipStream_t 
 // the chunk partials' workspace in floats (0 when one chunk covers the keys).
 struct AttnPlan {
   int gb = 1, splits = 1, chunk = 64;
+  int qtiles = 0;  // many query rows on the matrix cores (qnn_attention_mm.hip): 128-row tiles per KV head
   size_t part_floats = 0;
 };
-AttnPlan attn_plan(int rows, int heads, int kv_heads, int dim, int position, int window);
+AttnPlan attn_plan(int rows, int cap, int heads, int kv_heads, int dim, int position, int window);
+// Fills p (qtiles > 0) where the call takes the matrix cores; false otherwise.
+bool attn_mm_plan(AttnPlan &p, int rows, int cap, int heads, int kv_heads, int dim, int position, int window);
+void attn_mm_launch(const float *q, const float *cache, float *out, float *opart, float *ml, const AttnPlan &p, int rows,
+                    int cap, int heads, int kv_heads, int dim, int position, int window, float softcap, float scale,
+                    int masked, hipStream_t s);
 void attn_launch(const float *q, const float *cache, float *out, float *ws, const AttnPlan &p, int rows, int cap,
                  int heads, int kv_heads, int dim, int position, int window, float softcap, float scale, int masked,
                  hipStream_t s);

@@ -306,3 +306,91 @@ def test_gather_embedding_rows(ctx, rng, kind):
         ctx.Gather(td, ti, w, scales, ids.size, dim, vocab, 1)
     ctx.Recycle(ti)
     ctx.Recycle(td)
+
+
+MANY = [
+    # rows, heads, kvh, dim, cap, pos, window, softcap, scale, masked
+    (4, 4, 4, 64, 68, 64, 0, 0.0, 0.0, False),        # one head per KV head, four query rows of 128
+    (33, 28, 4, 80, 301, 268, 0, 0.0, 0.0, False),    # 7 heads per KV head, two row tiles; capacity no multiple of 4
+    (128, 8, 2, 128, 640, 500, 0, 0.0, 0.0, False),   # several workgroups per KV head
+    (40, 8, 2, 128, 200, 0, 0, 0.0, 0.0, False),      # from key 0: parts whose rows have no keys there
+    (17, 6, 2, 66, 130, 100, 0, 0.0, 0.0, False),     # dim no multiple of 4
+    (20, 4, 2, 33, 90, 60, 0, 0.0, 0.0, False),
+    (50, 16, 2, 96, 400, 333, 100, 0.0, 0.05, False),  # window, scale
+    (24, 8, 2, 128, 300, 200, 31, 30.0, 0.0, True),   # window shorter than a tile, soft cap, mask
+    (64, 4, 1, 64, 200, 100, 0, 20.0, 0.0, True),
+]
+
+
+def many_inputs(rng, case):
+    rows, heads, kvh, dim, cap, pos, _, _, _, masked = case
+    n = pos + rows
+    cache = np.zeros(2 * cap * kvh * dim + (rows * cap if masked else 0), np.float32)
+    # keys of very different sizes, tile by tile and within one
+    k = (rng.standard_normal((n, kvh, dim)) * np.exp2(rng.integers(-6, 2, (n, 1, 1)))).astype(np.float32)
+    v = (rng.standard_normal((n, kvh, dim)) * np.exp2(rng.integers(-12, 9, (n, 1, 1)))).astype(np.float32)
+    oracle.cache_write(cache, k, v, n, kvh, dim, cap, 0)
+    if n < cap:  # keys that no row sees yet may hold anything
+        junk = np.full((cap - n, kvh, dim), np.nan, np.float32)
+        oracle.cache_write(cache, junk, junk, cap - n, kvh, dim, cap, n)
+    if masked:
+        m = (rng.random((rows, cap)) < 0.6).astype(np.uint32)
+        m[:, :] |= (np.arange(cap)[None] == (pos + np.arange(rows))[:, None])  # its own key
+        cache.view(np.uint32)[2 * cap * kvh * dim:] = m.reshape(-1)
+    return (rng.standard_normal(rows * heads * dim)).astype(np.float32), cache
+
+
+@pytest.mark.parametrize("case", MANY, ids=[f"r{c[0]}h{c[1]}k{c[2]}d{c[3]}p{c[5]}w{c[6]}m{int(c[9])}" for c in MANY])
+def test_attention_of_many_rows(ctx, rng, tune, case):
+    """The matrix-core kernel (QNN_ATTN_MM=1: at any size) against the oracle and against k_attn (QNN_ATTN_MM=0).
+    Both hold 22 bits or more of every operand: scores off by 2^-21 of their terms, so p by that times the largest
+    |q k| sum (below 60 here), and the sums of p v by fp32's rounding: 1e-5 normwise."""
+    rows, heads, kvh, dim, cap, pos, window, softcap, scale, masked = case
+    q, cache = many_inputs(rng, case)
+    want = oracle.cached_attention(q, cache, rows, cap, heads, kvh, dim, pos, window, softcap, scale, masked)
+    want = want.reshape(rows * heads, dim)
+    tq, tc = up(ctx, q), up(ctx, cache)
+    got = {}
+    for name, mm, wgs in (("mm", "1", "512"), ("one part", "1", "1"), ("k_attn", "0", "512")):
+        tune("QNN_ATTN_MM", mm)
+        tune("QNN_ATTN_WGS", wgs)
+        to = ctx.UploadRaw(np.full(rows * heads * dim + 64, 7.0, np.float32))
+        ctx.CachedAttention(to, tq, tc, rows, cap, heads, kvh, dim, pos, window, softcap, scale, masked)
+        got[name] = ctx.Download(to)
+        assert np.all(got[name][rows * heads * dim:] == 7.0)
+        got[name] = got[name][:rows * heads * dim].reshape(rows * heads, dim)
+        ctx.Recycle(to)
+    for i in range(rows * heads):
+        assert normwise_rel_err(got["mm"][i], want[i]) <= 1e-5, i
+        assert normwise_rel_err(got["one part"][i], want[i]) <= 1e-5, i
+        assert normwise_rel_err(got["mm"][i], got["k_attn"][i]) <= 1e-5, i
+    for z in (tq, tc):
+        ctx.Recycle(z)
+
+
+@pytest.mark.parametrize("where", ["k", "v"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_attention_of_many_rows_infinite_keys(ctx, rng, tune, where, value):
+    """An infinity or NaN in one key reaches the rows that see it as it does in k_attn, and no other row."""
+    case = (48, 8, 2, 128, 200, 100, 0, 0.0, 0.0, False)
+    rows, heads, kvh, dim, cap, pos, window, softcap, scale, masked = case
+    q, cache = many_inputs(rng, case)
+    at = pos + 20  # rows 20 and later see it
+    if where == "k":
+        cache[(1 * dim + 5) * cap + at] = value
+    else:
+        cache[cap * kvh * dim + (1 * cap + at) * dim + 5] = value
+    tq, tc, to = up(ctx, q), up(ctx, cache), ctx.NewTensor(rows * heads * dim)
+    got = {}
+    for mm in ("1", "0"):
+        tune("QNN_ATTN_MM", mm)
+        ctx.CachedAttention(to, tq, tc, rows, cap, heads, kvh, dim, pos, window, softcap, scale, masked)
+        got[mm] = ctx.Download(to).reshape(rows, heads, dim)
+    a, b = got["1"], got["0"]
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isposinf(a), np.isposinf(b))
+    assert np.array_equal(np.isneginf(a), np.isneginf(b)) and np.all(np.isfinite(a[:20]))
+    assert not np.all(np.isfinite(b[20:]))
+    fine = np.isfinite(b)
+    assert np.max(np.abs(a[fine] - b[fine])) <= 1e-5 * np.max(np.abs(b[fine]))
+    for z in (tq, tc, to):
+        ctx.Recycle(z)
