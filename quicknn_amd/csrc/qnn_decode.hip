@@ -866,13 +866,19 @@ __global__ __launch_bounds__(256) void k_attn_merge_general(float *out, const fl
 // picks them (its running best starts there).
 //
 // Level 0 reads the logits and seen flags; a workgroup takes the exact top-k
-// of its 4096 tokens.  Each wave ranks its own 1024: a threshold found by
-// bisection over ballot counts keeps only the tokens that can be in the
-// wave's top-k (at least k half-lane maxima reach it), those are compacted,
-// and k rounds of a DPP wave-wide maximum rank them; wave 0 then ranks the
-// four waves' lists.  Levels above read the previous level's keys.  When a
-// level's keys fit one workgroup (tiles * k <= 4096) the last workgroup to
-// finish ranks them and draws the token (tensor.comp:177-197).
+// of its 4096 tokens: each wave bisects, over ballot counts, to a score that
+// at least k of its half-lane maxima reach; the keys that reach the highest of
+// the four waves' scores (about 4 k of them) are compacted into LDS, and each
+// one's rank is the number of larger keys.  Levels above read the previous
+// level's keys.  When a level's keys fit one workgroup (tiles * k <= 4096) the
+// last workgroup to finish ranks them and draws the token (tensor.comp:177-197).
+//
+// What bounds it: one chain of latencies (the loads, two rankings, the ticket),
+// on few CUs.  So the loads have no branches between them (in flight at once),
+// a ranking has three barriers, and the draw's running sums, which are to be
+// added in rank order, are one chain of k additions with a candidate per lane.
+// 151936 tokens, k = 40: 15 us (a bitonic sort per wave, a second one of the
+// four waves' lists, and the draw in one thread: 30).
 constexpr int kSampleThreads = 256;
 constexpr int kSamplePerThread = 16;
 constexpr int kSampleTile = kSampleThreads * kSamplePerThread;
@@ -940,168 +946,128 @@ __device__ __forceinline__ void rank_rounds(const uint64_t (&c)[J], int k, uint6
   }
 }
 
-template <int J>
-__device__ __forceinline__ void rank_from(const uint64_t *scratch, int count, int k, uint64_t *out) {
-  const int lane = threadIdx.x & 63;
-  uint64_t c[J];
-#pragma unroll
-  for (int i = 0; i < J; ++i) c[i] = i * 64 + lane < count ? scratch[i * 64 + lane] : 0ull;
-  rank_rounds<J>(c, k, out);
-}
-
-__device__ __forceinline__ uint64_t shfl_xor_key(uint64_t v, int m) {
-  const int lo = __shfl_xor(int(uint32_t(v)), m), hi = __shfl_xor(int(uint32_t(v >> 32)), m);
-  return (uint64_t(uint32_t(hi)) << 32) | uint32_t(lo);
-}
-
-// Sorts the wave's 64*J keys (element j*64 + lane in c[j]) into descending
-// order with a bitonic network, then writes ranks 0..k-1 (keys at or below the
-// floor become the floor).
-template <int J>
-__device__ __forceinline__ void sort_from(const uint64_t *scratch, int count, int k, uint64_t *out) {
-  const int lane = threadIdx.x & 63;
-  uint64_t c[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) c[j] = j * 64 + lane < count ? scratch[j * 64 + lane] : 0ull;
-#pragma unroll
-  for (int size = 2; size <= 64 * J; size <<= 1) {
-#pragma unroll
-    for (int stride = size / 2; stride > 0; stride >>= 1) {
-      if (stride >= 64) {
-        const int rs = stride / 64;
-#pragma unroll
-        for (int j = 0; j < J; ++j)
-          if ((j & rs) == 0) {
-            const int e = j * 64 + lane;
-            const bool desc = (e & size) == 0;
-            const uint64_t a = c[j], b = c[j | rs];
-            const uint64_t hi = a > b ? a : b, lo = a > b ? b : a;
-            c[j] = desc ? hi : lo;
-            c[j | rs] = desc ? lo : hi;
-          }
-      } else {
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-          const int e = j * 64 + lane;
-          const uint64_t other = shfl_xor_key(c[j], stride);
-          const bool desc = (e & size) == 0, first = (lane & stride) == 0;
-          const uint64_t hi = c[j] > other ? c[j] : other, lo = c[j] > other ? other : c[j];
-          c[j] = (first == desc) ? hi : lo;
-        }
-      }
-    }
-  }
-  const uint64_t floor = floor_key();
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int e = j * 64 + lane;
-    if (e < k) out[e] = c[j] > floor ? c[j] : floor;
-  }
-  if (lane == 0)
-    for (int e = 64 * J; e < k; ++e) out[e] = floor;
-}
-
-// Ranked top-k (k <= 64) of the wave's keys, N per lane, into out[0..k)
-// (unfilled ranks get floor_key()).  scratch: 64 * N keys of LDS.
-template <int N>
-__device__ __forceinline__ void wave_topk(const uint64_t (&key)[N], int k, uint64_t *scratch, uint64_t *out) {
-  const int lane = threadIdx.x & 63;
-  if (k <= 2) {  // a round or two of the wave-wide maximum beats filtering
-    rank_rounds<N>(key, k, out);
-    return;
-  }
-  // Threshold: the largest T with at least k half-lane maxima whose score
-  // bits reach T; every key of the top-k has score bits >= T.
-  uint32_t hm0 = 0, hm1 = 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const uint32_t h = uint32_t(key[i] >> 32);
-    if (i < (N + 1) / 2) hm0 = max(hm0, h);
-    else hm1 = max(hm1, h);
-  }
-  uint32_t t = 0;
-  for (int bit = 31; bit >= 0; --bit) {
-    const uint32_t c = t | (1u << bit);
-    const int n = __popcll(__ballot(hm0 >= c)) + (N > 1 ? __popcll(__ballot(hm1 >= c)) : 0);
-    if (n >= k) t = c;
-  }
-  // Compact the keys that reach it.
-  int count = 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const bool keep = key[i] != 0ull && uint32_t(key[i] >> 32) >= t;
-    const uint64_t mask = __ballot(keep);
-    if (keep) scratch[count + __popcll(mask & ((1ull << lane) - 1ull))] = key[i];
-    count += __popcll(mask);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // Few survivors (the usual case): sort them.  Many (ties, flat logits):
-  // k rounds of the wave-wide maximum.
-  const int per_lane = (count + 63) / 64;
-  if (per_lane <= 1)
-    sort_from<1>(scratch, count, k, out);
-  else if (per_lane <= 2)
-    sort_from<2>(scratch, count, k, out);
-  else if (per_lane <= 4 || N <= 4)
-    sort_from<(N < 4 ? N : 4)>(scratch, count, k, out);
-  else if (per_lane <= 8 || N <= 8)
-    rank_from<(N < 8 ? N : 8)>(scratch, count, k, out);
-  else
-    rank_from<N>(scratch, count, k, out);
-}
-
 struct SampleArgs {
   int count, k, tiles, level0, merge;
   float temperature, top_p, penalty, uniform;
 };
 
-// The workgroup's ranked top-k of its 4096 keys (16 per lane) into top[0..k).
-__device__ __forceinline__ void group_topk(const uint64_t (&key)[kSamplePerThread], int k, uint64_t *scratch,
-                                           uint64_t (*lists)[64], uint64_t *top) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  wave_topk<kSamplePerThread>(key, k, scratch + wave * 64 * kSamplePerThread, lists[wave]);
-  __syncthreads();
-  if (wave == 0) {
-    uint64_t c4[4];
+// Keys that are ranked by counting; more (ties, flat logits) are first cut to
+// each wave's own top-k by k rounds of the wave-wide maximum.  Counting costs
+// count x ceil(count / 256) LDS reads: 512 are about as long as 64 rounds.
+constexpr int kSampleCap = 512;
+struct SampleShared {
+  uint64_t cand[kSampleCap];
+  uint32_t t[4];
+  int count;
+};
+
+// The workgroup's ranked top-k (k <= 64) of its 4096 keys (16 per lane):
+// put(rank, key) for every rank below k, from one thread each.
+template <typename Put>
+__device__ __forceinline__ void group_topk(const uint64_t (&key)[kSamplePerThread], int k, SampleShared &sh, Put put) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t floor = floor_key();
+  // The largest t with at least k half-lane maxima whose score bits reach it
+  // (0: fewer than k): every key of the wave's top-k reaches t, and every key
+  // of the workgroup's top-k reaches each wave's t.
+  uint32_t hm0 = 0, hm1 = 0;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) c4[w] = lane < k ? lists[w][lane] : 0ull;
-    wave_topk<4>(c4, k, scratch, top);
+  for (int i = 0; i < kSamplePerThread; ++i) {
+    const uint32_t h = uint32_t(key[i] >> 32);
+    if (i < kSamplePerThread / 2) hm0 = max(hm0, h);
+    else hm1 = max(hm1, h);
   }
+  uint32_t t = 0;
+#pragma unroll 1
+  for (int bit = 31; bit >= 0; --bit) {
+    const uint32_t c = t | (1u << bit);
+    if (__popcll(__ballot(hm0 >= c)) + __popcll(__ballot(hm1 >= c)) >= k) t = c;
+  }
+  if (lane == 0) sh.t[wave] = t;
+  if (tid == 0) sh.count = 0;
+  __syncthreads();
+  t = max(max(sh.t[0], sh.t[1]), max(sh.t[2], sh.t[3]));
+  uint32_t keep = 0;
+  int mine = 0;
+#pragma unroll
+  for (int i = 0; i < kSamplePerThread; ++i) {
+    const bool in = key[i] > floor && uint32_t(key[i] >> 32) >= t;
+    keep |= uint32_t(in) << i;
+    mine += __popcll(__ballot(in));
+  }
+  int base = 0;
+  if (lane == 0) base = atomicAdd(&sh.count, mine);
+  base = __builtin_amdgcn_readfirstlane(base);
+  if (base + mine <= kSampleCap) {
+#pragma unroll
+    for (int i = 0; i < kSamplePerThread; ++i) {
+      const bool in = (keep >> i) & 1u;
+      const uint64_t mask = __ballot(in);
+      if (in) sh.cand[base + __popcll(mask & ((1ull << lane) - 1ull))] = key[i];
+      base += __popcll(mask);
+    }
+  }
+  __syncthreads();
+  int count = sh.count, above = count;
+  if (count > kSampleCap) {  // the same in every thread
+    __syncthreads();
+    rank_rounds<kSamplePerThread>(key, k, sh.cand + wave * k);
+    count = 4 * k;
+    __syncthreads();
+    above = 0;  // the lists end in floors
+    for (int j = 0; j < count; ++j) above += sh.cand[j] > floor;
+  }
+  for (int c = tid; c < count; c += kSampleThreads) {
+    const uint64_t v = sh.cand[c];
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < count; ++j) rank += sh.cand[j] > v;
+    if (rank < k && v > floor) put(rank, v);  // keys above the floor are distinct
+  }
+  if (tid < k && tid >= above) put(tid, floor);  // ranks that no key took
   __syncthreads();
 }
 
 __global__ __launch_bounds__(kSampleThreads) void k_sample(unsigned *dst, const float *logits, const unsigned *seen,
                                                            const uint64_t *in_keys, uint64_t *out_keys,
                                                            unsigned *counter, SampleArgs a) {
-  __shared__ uint64_t scratch[4 * 64 * kSamplePerThread];
-  __shared__ uint64_t lists[4][64];
+  __shared__ SampleShared sh;
   __shared__ uint64_t top[64];
-  __shared__ float top_w[64];
-  __shared__ unsigned ids[64];
   __shared__ unsigned last;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, tile = blockIdx.x;
   uint64_t key[kSamplePerThread];
-  // Wave w holds items [w*1024, (w+1)*1024) of the tile, lane-strided.
+  // Wave w holds items [w*1024, (w+1)*1024) of the tile, lane-strided.  Items
+  // past the end read the last one and give no key.
+  const unsigned item0 = unsigned(tile) * kSampleTile + unsigned(wave) * 1024 + lane;
+  const unsigned end = unsigned(a.count) - 1u;
+  if (a.level0) {
+    unsigned flag[kSamplePerThread];
+    float score[kSamplePerThread];
 #pragma unroll
-  for (int i = 0; i < kSamplePerThread; ++i) {
-    const unsigned item = unsigned(tile) * kSampleTile + unsigned(wave) * 1024 + unsigned(i) * 64 + lane;
-    key[i] = 0ull;
-    if (item < unsigned(a.count)) {
-      if (a.level0) {
-        const unsigned flag = seen[item];
-        float score = logits[item];
-        if (flag != 0u) score = score < 0.0f ? score * a.penalty : score / a.penalty;
-        key[i] = flag != kNoToken ? rank_key(score, item) : 0ull;
-      } else {
-        key[i] = __hip_atomic_load(&in_keys[item], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+    for (int i = 0; i < kSamplePerThread; ++i) {
+      const unsigned item = min(item0 + unsigned(i) * 64, end);
+      flag[i] = seen[item];
+      score[i] = logits[item];
     }
+#pragma unroll
+    for (int i = 0; i < kSamplePerThread; ++i) {
+      const unsigned item = item0 + unsigned(i) * 64;
+      float v = score[i];
+      if (flag[i] != 0u) v = v < 0.0f ? v * a.penalty : v / a.penalty;
+      key[i] = item <= end && flag[i] != kNoToken ? rank_key(v, item) : 0ull;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kSamplePerThread; ++i)
+      key[i] = __hip_atomic_load(&in_keys[min(item0 + unsigned(i) * 64, end)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int i = 0; i < kSamplePerThread; ++i)
+      if (item0 + unsigned(i) * 64 > end) key[i] = 0ull;
   }
-  group_topk(key, a.k, scratch, lists, top);
-  if (tid < a.k) __hip_atomic_store(&out_keys[size_t(tile) * a.k + tid], top[tid], __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT);
+  uint64_t *mine = out_keys + size_t(tile) * a.k;
+  group_topk(key, a.k, sh, [&](int rank, uint64_t v) {
+    __hip_atomic_store(&mine[rank], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  });
   if (!a.merge) return;
   // One ticket per workgroup once its keys are stored.
   __builtin_amdgcn_s_waitcnt(0);
@@ -1114,46 +1080,41 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(unsigned *dst, const 
   // The last workgroup ranks every tile's keys (at most 4096).
   const int count = a.tiles * a.k;
 #pragma unroll
-  for (int i = 0; i < kSamplePerThread; ++i) {
-    const int c = wave * 1024 + i * 64 + lane;
-    key[i] = c < count ? __hip_atomic_load(&out_keys[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-  }
-  group_topk(key, a.k, scratch, lists, top);
-  if (tid == 0) {
+  for (int i = 0; i < kSamplePerThread; ++i)
+    key[i] = __hip_atomic_load(&out_keys[min(wave * 1024 + i * 64 + lane, count - 1)], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int i = 0; i < kSamplePerThread; ++i)
+    if (wave * 1024 + i * 64 + lane >= count) key[i] = 0ull;
+  group_topk(key, a.k, sh, [&](int rank, uint64_t v) { top[rank] = v; });
+  if (wave == 0) {
 #pragma clang fp contract(off)
-    const uint64_t floor = floor_key();
-    for (int j = 0; j < a.k; ++j) {
-      const bool none = top[j] <= floor;
-      top_w[j] = none ? kLowest : from_order_bits(uint32_t(top[j] >> 32));
-      ids[j] = none ? kNoToken : ~uint32_t(top[j]);
-    }
-    unsigned selected = ids[0];
+    const uint64_t v = lane < a.k ? top[lane] : 0ull;
+    const bool none = v <= floor_key();
+    const float w = none ? kLowest : from_order_bits(uint32_t(v >> 32));
+    const unsigned id = none ? kNoToken : ~uint32_t(v);
+    int pick = 0;
     if (a.temperature > 0.0f && a.k > 1) {
-      float total = 0.0f;
-      const float maximum = top_w[0];
+      const float maximum = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), 0));
+      const float e = expf((w - maximum) / a.temperature);
+      // The sums up to each candidate, added in rank order.
+      float total = 0.0f, upto = 0.0f;
       for (int j = 0; j < a.k; ++j) {
-        top_w[j] = expf((top_w[j] - maximum) / a.temperature);
-        total += top_w[j];
+        total += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), j));
+        if (lane == j) upto = total;
       }
-      float retained = 0.0f;
-      int n = 0;
-      do {
-        retained += top_w[n];
-        ++n;
-      } while (n < a.k && retained < a.top_p * total);
-      const float target = a.uniform * retained;
-      float accumulated = 0.0f;
-      selected = ids[n - 1];
-      for (int j = 0; j < n; ++j) {
-        accumulated += top_w[j];
-        if (target < accumulated) {
-          selected = ids[j];
-          break;
-        }
-      }
+      // The first n whose sum reaches top_p of all, one at least.
+      const uint64_t below = __ballot(lane < a.k - 1 && upto < a.top_p * total);
+      const int n = __builtin_ctzll(~below) + 1;
+      const float target = a.uniform * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(upto), n - 1));
+      const uint64_t hit = __ballot(lane < n && target < upto);
+      pick = hit ? __builtin_ctzll(hit) : n - 1;
     }
-    dst[0] = selected;
-    dev::reset_counter(counter, 0);
+    const unsigned selected = unsigned(__builtin_amdgcn_readlane(int(id), pick));
+    if (tid == 0) {
+      dst[0] = selected;
+      dev::reset_counter(counter, 0);
+    }
   }
 }
 

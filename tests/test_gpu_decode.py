@@ -394,3 +394,33 @@ def test_attention_of_many_rows_infinite_keys(ctx, rng, tune, where, value):
     assert np.max(np.abs(a[fine] - b[fine])) <= 1e-5 * np.max(np.abs(b[fine]))
     for z in (tq, tc, to):
         ctx.Recycle(z)
+
+
+@pytest.mark.parametrize("vocab,k,levels", [
+    (1, 1, 0), (63, 64, 0), (4095, 64, 0), (4097, 40, 3), (8192, 3, 0), (9000, 64, 1), (20000, 64, 1), (20000, 33, 40),
+    (263000, 64, 0), (263000, 64, 2)])
+def test_sampling_ranks_at_edges(ctx, rng, vocab, k, levels):
+    """Every rank of the list, at the edges of tiles, of the counting (512 keys that reach the threshold) and of the
+    levels (tiles x k of 4096); `levels` distinct scores only (0: all distinct; 1: everything tied), and infinities,
+    NaNs and the lowest score among them."""
+    if levels:
+        logits = rng.integers(0, levels, vocab).astype(np.float32)
+    else:
+        logits = rng.permutation(vocab).astype(np.float32) - vocab // 2
+    seen = np.zeros(vocab, np.uint32)
+    seen[rng.random(vocab) < 0.1] = 0xFFFFFFFF
+    seen[rng.integers(0, vocab)] = 0
+    special = rng.permutation(vocab)[:min(vocab // 50, 40)]
+    for j, v in enumerate((np.nan, -np.inf, np.float32(-3.402823466e38), 0.0, -0.0)):
+        logits[special[j::5]] = v
+    tl, ts = up(ctx, logits), up(ctx, seen)
+    kk = min(k, vocab)
+    alive = np.flatnonzero((seen != 0xFFFFFFFF) & ~np.isnan(logits) & (logits > -3.402823466e38))
+    order = alive[np.lexsort((alive, -logits[alive].astype(np.float64)))][:kk]
+    # So high a temperature that every token weighs the same (expf of -2e-33 or so is 1), and the ranks that no token
+    # takes, as -FLT_MAX, expf(-3.4028...): u picks the rank.
+    total = len(order) + (kk - len(order)) * np.exp(-3.402823466)
+    for j in sorted({0, 1, 2, kk // 2, kk - 2, kk - 1} & set(range(len(order)))):
+        assert sample(ctx, logits, seen, kk, 1e38, 1.0, 1.0, (j + 0.5) / total, tl, ts) == int(order[j]), j
+    ctx.Recycle(tl)
+    ctx.Recycle(ts)
