@@ -73,6 +73,24 @@ def test_fp16_copy_equals_decoding_kernel(ctx, rng, tune, m, k, n):
         assert normwise_rel_err(fast[r], oracle.cpu_linear(w, ENC_Q8_0, a[r], k, n)) <= TOL, r
 
 
+@pytest.mark.parametrize("m,n", [(128, 4), (129, 188), (160, 192), (255, 196), (128, 191), (130, 194), (200, 388)])
+def test_fp16_copy_output_edges(ctx, rng, tune, m, n):
+    """Rows and columns that end inside a 128 x 192 tile, rows of C of whole 16 bytes and not: the same bits as the
+    decoding kernel, and nothing written past C."""
+    k = 64
+    src, dst = ctx.UploadRaw(rng.standard_normal((m, k)).astype(np.float32)), None
+    blk = hip.MemoryBlock.gguf(q8(rng, n, k), n, k, ENC_Q8_0)
+    got = []
+    for rows in ("128", "0"):
+        tune("QNN_GEMM_H16", rows)
+        dst = ctx.UploadRaw(np.full(m * n + 256, 7.0, np.float32))
+        ctx.Linear(dst, src, blk, None, None, m, k, n)
+        got.append(ctx.Download(dst))
+        ctx.Recycle(dst)
+    assert np.array_equal(got[0], got[1]) and np.all(got[0][m * n:] == 7.0) and not np.any(got[0][:m * n] == 7.0)
+    ctx.Recycle(src)
+
+
 @pytest.mark.parametrize("enc", [ENC_Q8_0, ENC_Q4_K])
 def test_rows_in_several_gemm_launches(ctx, rng, tune, enc):
     """Rows beyond one launch's limit run as consecutive launches (the limit keeps the activation
