@@ -1026,9 +1026,22 @@ int gemm_max_rows(int in_dim) {
   return int(std::min<size_t>(m, size_t(1) << 30));
 }
 
-// Multi-row GGUF projection.  From QNN_GEMM_H16 rows (Q8_0) or
-// QNN_GGUF_GEMM_ROWS rows (the other encodings): k_h16_gemm over the weight's
-// fp16 copy; otherwise, and under capture while no copy exists, a Q8_0 weight
+// Fewer rows than QNN_GEMM_H16 (from q8_gemm_min_rows on) take the fp16 copy
+// too where it is there or costs no other weight its place: 8 rows of 3072 ->
+// 12288 take 18.0 us over the copy, 36.5 decoding; of 4096 -> 4096 19.5 and
+// 49.7; 64 rows 19.1 and 39.1, 20.4 and 52.0.  Weights below 1 M elements keep
+// decoding: their copy takes longer to make (30 us and more) than a few such
+// calls save (1024 -> 1000: 10.6 and 18.9).  The results are the same bits.
+bool few_rows_take_copy(qnn_ctx_s *ctx, const WeightEntry *w, int rows, size_t copy_bytes) {
+  if (w->gg.enc != QNN_WE_Q8_0 || tuning().gemm_h16 <= 0 || rows < q8_gemm_min_rows() ||
+      int64_t(w->gg.rows) * w->gg.cols < (1 << 20))
+    return false;
+  return ctx->weight_bytes + copy_bytes <= ctx->weight_limit || ctx->weights.count(w->key + "/h16") != 0;
+}
+
+// Multi-row GGUF projection.  From QNN_GEMM_H16 rows (Q8_0; fewer:
+// few_rows_take_copy) or QNN_GGUF_GEMM_ROWS rows (the other encodings):
+// k_h16_gemm over the weight's fp16 copy; otherwise, and under capture while no copy exists, a Q8_0 weight
 // from q8_gemm_min_rows rows takes k_q8_gemm, which decodes its tiles.  False
 // when neither applies: the caller then runs the matvec, up to kGGMaxTokens
 // rows per pass.  (Measured with the GEMM's K-slices: at 8 rows the matvec is
@@ -1042,7 +1055,7 @@ bool run_gguf_gemm(qnn_ctx_s *ctx, WeightEntry *w, const float *x, float *y, int
   // activation fragments with 32-bit buffer offsets: larger weights take the
   // matvec, and the caller passes at most gemm_max_rows rows.
   const size_t copy_bytes = q8_h16_bytes(w->gg.rows, w->gg.cols) + (size_t(w->gg.rows) * 4 + 255) / 256 * 256;
-  if (from > 0 && rows >= from && copy_bytes <= 0xFFFFFFFFull) {
+  if (from > 0 && (rows >= from || few_rows_take_copy(ctx, w, rows, copy_bytes)) && copy_bytes <= 0xFFFFFFFFull) {
     w->op_pins++;  // making the copy may evict: not the weight it is made from
     WeightEntry *h = nullptr;
     try {
@@ -1056,16 +1069,15 @@ bool run_gguf_gemm(qnn_ctx_s *ctx, WeightEntry *w, const float *x, float *y, int
       const int *ew = q8 ? reinterpret_cast<const int *>(static_cast<const uint8_t *>(w->dptr) + w->gg.rowexp_off)
                          : reinterpret_cast<const int *>(static_cast<const uint8_t *>(h->dptr) +
                                                          q8_h16_bytes(w->gg.rows, w->gg.cols));
-      const Q8GemmPlan p = q8_h16_plan(rows, in_dim, out_dim);
       // Small grids split K (the other encodings only: a Q8_0 copy's product
       // stays bit-identical to the decoding kernel's).
-      const int ksplit = q8 ? 1 : h16_ksplit(p, out_dim);
+      const Q8GemmPlan p = h16_plan(rows, in_dim, out_dim, !q8);
       const size_t frag_off = 0, exp_off = (p.frag_bytes + 255) & ~size_t(255);
       const size_t part_off = (exp_off + p.exp_bytes + 255) & ~size_t(255);
-      const size_t part_bytes = ksplit > 1 ? size_t(ksplit) * rows * out_dim * 4 : 0;
+      const size_t part_bytes = p.ksplit > 1 ? size_t(p.ksplit) * rows * out_dim * 4 : 0;
       uint8_t *ws = static_cast<uint8_t *>(ensure_work(ctx, part_off + part_bytes));
       q8_h16_gemm_launch(p, x, rows, in_dim, out_dim, ew, h->dptr, ws + frag_off,
-                         reinterpret_cast<int *>(ws + exp_off), y, ctx->stream, ksplit,
+                         reinterpret_cast<int *>(ws + exp_off), y, ctx->stream,
                          reinterpret_cast<float *>(ws + part_off));
       ctx->st.gemm_h16++;
       return true;

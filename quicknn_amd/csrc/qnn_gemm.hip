@@ -394,32 +394,48 @@ __global__ __launch_bounds__(256) void k_q8_expand_h16(GGLayout l, const uint8_t
   out[idx] = v;
 }
 
-// Workgroup tile 128 x 192 (a 512 x 12288 product is 4 x 64 = 256
-// workgroups, one per CU), four waves of 64 x 96 (2 x 3 MFMA tiles), K-tiles
-// of 64.  A K-tile's fragments (A: 4 x 4 pieces, B: 6 x 4 pieces of 1 KiB)
-// go from global memory straight into LDS (buffer_load ... lds: each lane's
-// 16 bytes land at M0 + 16 lane, so a piece keeps its [lane] order) through
-// HST stages of 40 KiB (all 160 KiB of the CU's LDS: the loads run up to
-// three K-tiles ahead).  Per K-tile, one barrier: after it the K-tile's stage
-// is free (every wave holds its fragments in registers) and takes the loads
-// of K-tile kt + HST; then each wave reads the next K-tile's fragments (20
-// pieces, 80 VGPRs) while its MFMAs run on the current ones.  Per 32 x 32
-// tile the MFMAs run over K in order, as in k_q8_gemm, so C is the same, bit
-// for bit.
-constexpr int HBM = 128, HBN = 192, HKT = 4;  // rows, columns, K-steps (of 16) per K-tile
-constexpr int HAP = HBM / 32 * HKT, HBP = HBN / 32 * HKT;  // 1 KiB pieces per K-tile: 16 + 24
-constexpr int HPW = (HAP + HBP) / 4;                        // pieces each wave loads per K-tile: 10
-constexpr int HLD = HBN + 8;                                // floats per LDS row of C (the two half-waves' rows 32 banks apart)
-constexpr int HST = 4;                                      // LDS stages
-constexpr size_t kH16Lds = size_t(HST) * (HAP + HBP) * 1024;
-static_assert(HAP % 4 == 0 && kH16Lds <= 160 * 1024, "h16 tiling");
+// A workgroup is four waves over a tile of 32 MB x 32 NB of C, WM of them along
+// the rows, with K-tiles of 64.  A K-tile's fragments (A: MB x 4 pieces of 1
+// KiB, B: NB x 4) go from global memory straight into LDS (buffer_load ...
+// lds: each lane's 16 bytes land at M0 + 16 lane, so a piece keeps its [lane]
+// order) through ST stages: the loads run up to ST - 1 K-tiles ahead.  Per
+// K-tile, one barrier: after it the K-tile's stage is free (every wave holds
+// its fragments in registers) and takes the loads of K-tile kt + ST; then each
+// wave reads the next K-tile's fragments while its MFMAs run on the current
+// ones.  Per 32 x 32 tile the MFMAs run over K in order, as in k_q8_gemm, so
+// C is the same, bit for bit, in every shape.
+//
+// The shapes (h16_plan picks one) differ in how many rows are padded, how many
+// workgroups there are, and what a K-tile costs; every shape takes 25-30 bytes
+// per clock and workgroup from L2, whatever its depth (eight stages of 32 x 128
+// 0.38 us per K-tile, four 0.41), so a larger tile does more per byte:
+//   128 x 192 (wave 64 x 96), 160 KiB: 0.66 us per K-tile; 512 x 12288 is 256
+//       workgroups, one per CU;
+//   128 x 128 (64 x 64), 160 KiB: 0.58; 200 rows of 3584 -> 14336 40 us (128 x
+//       192: 150 workgroups, 45);
+//   64 x 128 (32 x 64), two workgroups per CU: 0.48 alone, 0.75 both;
+//   32 x 128 (32 x 32), two per CU: 0.41, 0.47; 16 rows of 3584 -> 14336 21.5
+//       us in two K-slices, 29.8 unsliced (128 x 192: 43.7).
+constexpr int HKT = 4;        // K-steps (of 16) per K-tile
+constexpr int kH16Pad = 192;  // the copy's rows are padded to this
+template <int MB_, int NB_, int WM_, int ST_>
+struct H16Shape {
+  static constexpr int MB = MB_, NB = NB_, WM = WM_, ST = ST_;
+  static constexpr int BM = 32 * MB, BN = 32 * NB, WN = 4 / WM;
+  static constexpr int TM = MB / WM, TN = NB / WN;       // MFMA tiles of a wave
+  static constexpr int AP = MB * HKT, BP = NB * HKT;     // 1 KiB pieces per K-tile
+  static constexpr int PW = MB + NB;                     // pieces each wave loads per K-tile
+  static constexpr int LD = BN + 8;                      // floats per LDS row of C (the two half-waves' rows 32 banks apart)
+  static constexpr size_t lds = size_t(ST) * (AP + BP) * 1024;
+  static_assert(MB % WM == 0 && NB % WN == 0 && HKT == 4 && lds <= 160 * 1024 && size_t(BM) * LD * 4 <= lds, "h16 shape");
+};
 struct H16Args {
   const uint4 *afrag;  // [m_pad / 32][ksteps][64]
   const int *ea;
   const uint4 *wfrag;  // [n_pad / 32][ksteps][64]
   const int *ew;       // [rows] weight row exponents
   float *c;            // ksplit 1: C [M][N]; else the slices' partial products [ksplit][M][N]
-  int M, N, ksteps, ktiles, mtiles, ntiles, ksplit;
+  int M, N, ksteps, ktiles, mtiles, ntiles, ksplit, nblocks;  // nblocks: 32-row blocks of the copy
 };
 
 // One 1 KiB piece from global memory into LDS at `lds` (wave-uniform).  The
@@ -439,15 +455,16 @@ __device__ __forceinline__ void h16_vmwait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-extern __shared__ uint4 h16_lds[];  // HST stages of [HAP + HBP] pieces: A [m32][ks], then B [n32][ks]
+extern __shared__ uint4 h16_lds[];  // ST stages of [AP + BP] pieces: A [m32][ks], then B [n32][ks]
 
+template <typename S>
 struct H16Frags {
-  half8 a[HKT][2], b[HKT][3];
+  half8 a[HKT][S::TM], b[HKT][S::TN];
 };
 
 // KS: the launch slices K (g.ksplit > 1); the instance without slices keeps
 // the plain N-tile mapping and loop bounds.
-template <bool KS>
+template <typename S, bool KS>
 __global__ __launch_bounds__(256) void k_h16_gemm(const H16Args g) {
   const int b = blockIdx.x;
   // Units (N-tile, K-slice) are dealt to the XCDs in turn; the M-tiles of a
@@ -461,88 +478,93 @@ __global__ __launch_bounds__(256) void k_h16_gemm(const H16Args g) {
   const int kt0 = KS ? ks * g.ktiles / g.ksplit : 0;
   const int nkt = KS ? (ks + 1) * g.ktiles / g.ksplit - kt0 : g.ktiles;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % S::WM, wn = wave / S::WM;
 
-  const Rsrc ar = rsrc(g.afrag, size_t(g.mtiles) * (HBM / 32) * g.ksteps * 1024);
-  const Rsrc br = rsrc(g.wfrag, size_t(g.ntiles) * (HBN / 32) * g.ksteps * 1024);
+  const Rsrc ar = rsrc(g.afrag, size_t(g.mtiles) * S::MB * g.ksteps * 1024);
+  const Rsrc br = rsrc(g.wfrag, size_t(g.nblocks) * g.ksteps * 1024);
   const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(h16_lds));
-  // This wave loads pieces p = wave + 4 i of every K-tile: i < HAP / 4 are A pieces.
-  uint32_t voff[HPW];
+  // This wave loads pieces p = wave + 4 i of every K-tile, so K-step `wave` of
+  // the A blocks (i < MB), then of the B blocks; a block past the copy's (the
+  // last tile's) reads the copy's last one, for columns that are not written.
+  uint32_t voff[S::PW];
 #pragma unroll
-  for (int i = 0; i < HPW; ++i) {
-    const int p = wave + 4 * i;
-    if (i < HAP / 4) {
-      voff[i] = uint32_t(((size_t(mtile) * (HBM / 32) + p / HKT) * g.ksteps + p % HKT) * 1024 + lane * 16);
-    } else {
-      const int pb = p - HAP;
-      voff[i] = uint32_t(((size_t(ntile) * (HBN / 32) + pb / HKT) * g.ksteps + pb % HKT) * 1024 + lane * 16);
-    }
+  for (int i = 0; i < S::PW; ++i) {
+    const int blk = i < S::MB ? mtile * S::MB + i : min(ntile * S::NB + i - S::MB, g.nblocks - 1);
+    voff[i] = uint32_t((size_t(blk) * g.ksteps + wave) * 1024 + lane * 16);
   }
   auto dma = [&](int kt, int i) {
-    const uint32_t st = lds0 + uint32_t(kt % HST) * ((HAP + HBP) * 1024u);
-    h16_dma(i < HAP / 4 ? ar : br, __builtin_amdgcn_readfirstlane(st + uint32_t(wave + 4 * i) * 1024u), voff[i],
+    const uint32_t st = lds0 + uint32_t(kt % S::ST) * ((S::AP + S::BP) * 1024u);
+    h16_dma(i < S::MB ? ar : br, __builtin_amdgcn_readfirstlane(st + uint32_t(wave + 4 * i) * 1024u), voff[i],
             uint32_t(kt0 + kt) * (HKT * 1024u));
   };
-  // Piece r of this wave's 5 HKT per K-tile: K-step r / 5, then A rows wm*2 + 0..1, B columns wn*3 + 0..2.
-  auto read1 = [&](H16Frags &f, const uint4 *st, int r) {
-    const int ks = r / 5, j = r % 5;
-    if (j < 2)
-      __builtin_memcpy(&f.a[ks][j], &st[((wm * 2 + j) * HKT + ks) * 64 + lane], 16);
+  // Piece r of this wave's (TM + TN) HKT per K-tile: K-step r / (TM + TN), then its A rows, its B columns.
+  constexpr int RS = S::TM + S::TN, READS = RS * HKT, MFMAS = S::TM * S::TN * HKT;
+  auto read1 = [&](H16Frags<S> &f, const uint4 *st, int r) {
+    const int ks = r / RS, j = r % RS;
+    if (j < S::TM)
+      __builtin_memcpy(&f.a[ks][j], &st[((wm * S::TM + j) * HKT + ks) * 64 + lane], 16);
     else
-      __builtin_memcpy(&f.b[ks][j - 2], &st[(HAP + (wn * 3 + j - 2) * HKT + ks) * 64 + lane], 16);
+      __builtin_memcpy(&f.b[ks][j - S::TM], &st[(S::AP + (wn * S::TN + j - S::TM) * HKT + ks) * 64 + lane], 16);
   };
 
-  f32x16 acc[2][3];
+  f32x16 acc[S::TM][S::TN];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < S::TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
+    for (int j = 0; j < S::TN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
   // K-tile kt: wait for K-tile kt + 1 (this wave's pieces, then everybody's:
-  // K-tile kt's stage is then free), then the 24 MFMAs of K-tile kt, each
-  // followed by one read of K-tile kt + 1's fragments and every second one by
-  // one load of K-tile kt + HST into kt's stage, in this order (an MFMA does
-  // not wait behind the wave's memory instructions).
-  auto tile = [&](auto REFILL, const H16Frags &cur, H16Frags &nxt, int kt) {
+  // K-tile kt's stage is then free), then the MFMAs of K-tile kt, each followed
+  // by its share of the reads of K-tile kt + 1's fragments and of the loads of
+  // K-tile kt + ST into kt's stage, in this order (an MFMA does not wait behind
+  // the wave's memory instructions).
+  auto tile = [&](auto REFILL, const H16Frags<S> &cur, H16Frags<S> &nxt, int kt) {
     if (decltype(REFILL)::value)
-      h16_vmwait<HPW * (HST - 2)>();
+      h16_vmwait<S::PW * (S::ST - 2)>();
     else
       h16_vmwait<0>();
     __syncthreads();
-    const uint4 *st = h16_lds + ((kt + 1) % HST) * ((HAP + HBP) * 64);  // past the end: unused
+    const uint4 *st = h16_lds + ((kt + 1) % S::ST) * ((S::AP + S::BP) * 64);  // past the end: unused
+    constexpr int RJ = (READS + MFMAS - 1) / MFMAS;                              // reads after each MFMA
+    constexpr int DJ = (S::PW + MFMAS - 1) / MFMAS, DE = MFMAS >= 2 * S::PW ? 2 : 1;  // DJ loads after each DE'th
 #pragma unroll
-    for (int j = 0; j < 6 * HKT; ++j) {
-      const int ks = j / 6, mb = (j % 6) / 3, nb = j % 3;
+    for (int j = 0; j < MFMAS; ++j) {
+      const int ks = j / (S::TM * S::TN), mb = j % (S::TM * S::TN) / S::TN, nb = j % S::TN;
       acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.a[ks][mb], cur.b[ks][nb], acc[mb][nb], 0, 0, 0);
-      if (j < 5 * HKT) read1(nxt, st, j);
-      if (decltype(REFILL)::value && (j & 1) && j / 2 < HPW) dma(kt + HST, j / 2);
+#pragma unroll
+      for (int r = j * RJ; r < j * RJ + RJ; ++r)
+        if (r < READS) read1(nxt, st, r);
+      if (decltype(REFILL)::value && j % DE == DE - 1)
+#pragma unroll
+        for (int i = j / DE * DJ; i < j / DE * DJ + DJ; ++i)
+          if (i < S::PW) dma(kt + S::ST, i);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 #pragma unroll
-  for (int d = 0; d < HST; ++d)
+  for (int d = 0; d < S::ST; ++d)
     if (d < nkt)
 #pragma unroll
-      for (int i = 0; i < HPW; ++i) dma(d, i);
-  H16Frags f0, f1;
-  if (HST - 1 < nkt)
-    h16_vmwait<HPW * (HST - 1)>();
+      for (int i = 0; i < S::PW; ++i) dma(d, i);
+  H16Frags<S> f0, f1;
+  if (S::ST - 1 < nkt)
+    h16_vmwait<S::PW * (S::ST - 1)>();
   else
     h16_vmwait<0>();
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < 5 * HKT; ++r) read1(f0, h16_lds, r);
+  for (int r = 0; r < READS; ++r) read1(f0, h16_lds, r);
   using Y = std::true_type;
   using N = std::false_type;
   int kt = 0;
-  for (; kt + 1 + HST < nkt; kt += 2) {  // both K-tiles refill
+  for (; kt + 1 + S::ST < nkt; kt += 2) {  // both K-tiles refill
     tile(Y(), f0, f1, kt);
     tile(Y(), f1, f0, kt + 1);
   }
   for (; kt < nkt; kt += 2) {
-    if (kt + HST < nkt)
+    if (kt + S::ST < nkt)
       tile(Y(), f0, f1, kt);
     else
       tile(N(), f0, f1, kt);
@@ -560,46 +582,46 @@ __global__ __launch_bounds__(256) void k_h16_gemm(const H16Args g) {
   // and keeping the lines out of the L2 shortens that burst.  All of it takes
   // 3.1 us (512 x 12288: 3.5); 12.9 with conditional loads and 4-byte stores
   // under a branch each, 9.5 with those stores alone.
-  int ear[2][16], ewr[3];
+  int ear[S::TM][16], ewr[S::TN];
 #pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
+  for (int mb = 0; mb < S::TM; ++mb)
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      ear[mb][i] = g.ea[mtile * HBM + (wm * 2 + mb) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)];
+      ear[mb][i] = g.ea[mtile * S::BM + (wm * S::TM + mb) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)];
 #pragma unroll
-  for (int nb = 0; nb < 3; ++nb) ewr[nb] = g.ew[min(ntile * HBN + (wn * 3 + nb) * 32 + (lane & 31), g.N - 1)];
-  float *c = g.c + (size_t(ks) * g.M + size_t(mtile) * HBM) * g.N + ntile * HBN;
-  const int mrows = min(HBM, g.M - mtile * HBM), ncols = min(HBN, g.N - ntile * HBN);
+  for (int nb = 0; nb < S::TN; ++nb) ewr[nb] = g.ew[min(ntile * S::BN + (wn * S::TN + nb) * 32 + (lane & 31), g.N - 1)];
+  float *c = g.c + (size_t(ks) * g.M + size_t(mtile) * S::BM) * g.N + ntile * S::BN;
+  const int mrows = min(S::BM, g.M - mtile * S::BM), ncols = min(S::BN, g.N - ntile * S::BN);
   if (g.N % 4 == 0) {
     float *out = reinterpret_cast<float *>(h16_lds);
     __syncthreads();  // every wave's reads of the stages
 #pragma unroll
-    for (int nb = 0; nb < 3; ++nb)
+    for (int nb = 0; nb < S::TN; ++nb)
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < S::TM; ++mb)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          out[((wm * 2 + mb) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)) * HLD + (wn * 3 + nb) * 32 + (lane & 31)] =
+          out[((wm * S::TM + mb) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)) * S::LD + (wn * S::TN + nb) * 32 + (lane & 31)] =
               ldexpf(acc[mb][nb][i], ear[mb][i] + ewr[nb]);
     __syncthreads();
 #pragma unroll 8
-    for (int j = tid; j < HBM * (HBN / 4); j += 256) {
-      const int row = j / (HBN / 4), col = j % (HBN / 4) * 4;
+    for (int j = tid; j < S::BM * (S::BN / 4); j += 256) {
+      const int row = j / (S::BN / 4), col = j % (S::BN / 4) * 4;
       if (row < mrows && col < ncols) {
         typedef float f32x4 __attribute__((ext_vector_type(4)));
-        const f32x4 v = *reinterpret_cast<const f32x4 *>(&out[row * HLD + col]);
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(&out[row * S::LD + col]);
         __builtin_nontemporal_store(v, reinterpret_cast<f32x4 *>(&c[size_t(row) * g.N + col]));
       }
     }
   } else {
 #pragma unroll
-    for (int nb = 0; nb < 3; ++nb) {
-      const int col = (wn * 3 + nb) * 32 + (lane & 31);
+    for (int nb = 0; nb < S::TN; ++nb) {
+      const int col = (wn * S::TN + nb) * 32 + (lane & 31);
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < S::TM; ++mb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int row = (wm * 2 + mb) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+          const int row = (wm * S::TM + mb) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
           if (row < mrows && col < ncols) c[size_t(row) * g.N + col] = ldexpf(acc[mb][nb][i], ear[mb][i] + ewr[nb]);
         }
     }
@@ -609,7 +631,7 @@ __global__ __launch_bounds__(256) void k_h16_gemm(const H16Args g) {
 }  // namespace
 
 size_t q8_h16_bytes(int rows, int cols) {
-  const size_t n_pad = size_t((rows + HBN - 1) / HBN) * HBN, k_pad = size_t((cols + 63) / 64) * 64;
+  const size_t n_pad = size_t((rows + kH16Pad - 1) / kH16Pad) * kH16Pad, k_pad = size_t((cols + 63) / 64) * 64;
   return n_pad * k_pad * 2;
 }
 
@@ -621,13 +643,52 @@ void q8_expand_h16_launch(const GGLayout &l, const void *w, void *out, hipStream
   hip_check(hipGetLastError(), "q8 fp16 expansion");
 }
 
-Q8GemmPlan q8_h16_plan(int M, int K, int N) {
+namespace {
+using H16A = H16Shape<4, 6, 2, 4>;
+using H16B = H16Shape<4, 4, 2, 5>;
+using H16C = H16Shape<2, 4, 2, 3>;
+using H16D = H16Shape<1, 4, 1, 4>;
+// What a workgroup of each shape was measured to take: its fixed part (first
+// loads, output), and a K-tile with one workgroup on the CU or all it holds.
+struct H16Cost {
+  int bm, bn, per_cu;
+  float fixed, alone, full;  // us
+};
+constexpr H16Cost kH16Cost[] = {{H16A::BM, H16A::BN, 1, 7.3f, 0.66f, 0.66f},
+                                {H16B::BM, H16B::BN, 1, 6.3f, 0.58f, 0.58f},
+                                {H16C::BM, H16C::BN, 2, 4.5f, 0.48f, 0.75f},
+                                {H16D::BM, H16D::BN, 2, 4.0f, 0.41f, 0.47f}};
+}  // namespace
+
+// The shape and the K-slices (at most 8, of 6 K-tiles at least) with the
+// shortest time: rounds of workgroups on an XCD's 32 CUs, no less than the
+// copy's bytes take from memory (5 TB/s), plus the slices' sum (its launch,
+// and 4.8 TB/s).
+Q8GemmPlan h16_plan(int M, int K, int N, bool split) {
   Q8GemmPlan p;
-  p.m_pad = (M + HBM - 1) / HBM * HBM;
   p.k_pad = (K + 63) / 64 * 64;
   p.ksteps = p.k_pad / 16;
-  p.mtiles = p.m_pad / HBM;
-  p.ntiles = (N + HBN - 1) / HBN;
+  const int ktiles = p.ksteps / HKT;
+  const float copy_us = float(N) * p.k_pad * 0.4e-6f;
+  float best = 0.0f;
+  for (int i = 0; i < int(sizeof(kH16Cost) / sizeof(*kH16Cost)); ++i) {
+    const H16Cost &c = kH16Cost[i];
+    const int mtiles = (M + c.bm - 1) / c.bm, ntiles = (N + c.bn - 1) / c.bn;
+    for (int s = 1; s == 1 || (split && N % 4 == 0 && s <= 8 && ktiles / s >= 6); ++s) {
+      const int64_t wgs = int64_t((ntiles * s + 7) / 8) * mtiles;  // of an XCD
+      const int64_t rounds = (wgs + 32 * c.per_cu - 1) / (32 * c.per_cu);
+      const float gemm = float(rounds) * (c.fixed + float((ktiles + s - 1) / s) * (wgs <= 32 ? c.alone : c.full));
+      const float us = std::max(gemm, copy_us) + (s > 1 ? 2.5f + float(s + 1) * float(M) * float(N) * 0.83e-6f : 0.0f);
+      if (best == 0.0f || us < best) {
+        best = us;
+        p.shape = i;
+        p.ksplit = s;
+        p.mtiles = mtiles;
+        p.ntiles = ntiles;
+        p.m_pad = mtiles * c.bm;
+      }
+    }
+  }
   p.frag_bytes = size_t(p.m_pad) * p.k_pad * 2;
   p.exp_bytes = size_t(p.m_pad) * 4;
   return p;
@@ -649,48 +710,44 @@ __global__ __launch_bounds__(256) void k_sum_kslices(float4 *__restrict__ c, con
   c[i] = v;
 }
 
-// K-slices for a grid of few tiles: as many as keep every workgroup of the
-// launch resident at once.  The kernel takes a CU's whole LDS (one workgroup
-// per CU), and an XCD (32 CUs) holds ceil(ntiles * ksplit / 8) units of
-// mtiles workgroups; at least 8 K-tiles per slice, at most 8 slices.
-int h16_ksplit(const Q8GemmPlan &p, int N) {
-  const int ktiles = p.ksteps / HKT;
-  if (N % 4 != 0) return 1;
-  int best = 1;
-  for (int s = 2; s <= 8 && ktiles / s >= 8; ++s)
-    if ((p.ntiles * s + 7) / 8 * p.mtiles <= 32) best = s;
-  return best;
+namespace {
+template <typename S, bool KS>
+void h16_launch(const H16Args &g, hipStream_t s) {
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_h16_gemm<S, KS>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(S::lds));
+  hip_check(attr, "fp16-copy gemm LDS size");
+  const int grid = (g.ntiles * g.ksplit + 7) / 8 * 8 * g.mtiles;
+  hipLaunchKernelGGL((k_h16_gemm<S, KS>), dim3(grid), dim3(256), S::lds, s, g);
 }
+template <typename S>
+void h16_launch(const H16Args &g, hipStream_t s) {
+  g.ksplit > 1 ? h16_launch<S, true>(g, s) : h16_launch<S, false>(g, s);
+}
+}  // namespace
 
 void q8_h16_gemm_launch(const Q8GemmPlan &p, const float *a, int M, int K, int N, const int *ew, const void *w16,
-                        void *frag, int *ea, float *c, hipStream_t s, int ksplit, float *part) {
+                        void *frag, int *ea, float *c, hipStream_t s, float *part) {
   hipLaunchKernelGGL(k_act_prep, dim3(p.m_pad / 4), dim3(1024), 0, s, a, M, K, p.ksteps, ea, static_cast<uint4 *>(frag));
   H16Args g;
   g.afrag = static_cast<const uint4 *>(frag);
   g.ea = ea;
   g.wfrag = static_cast<const uint4 *>(w16);
   g.ew = ew;
-  g.c = ksplit > 1 ? part : c;
+  g.c = p.ksplit > 1 ? part : c;
   g.M = M;
   g.N = N;
   g.ksteps = p.ksteps;
   g.ktiles = p.ksteps / HKT;
   g.mtiles = p.mtiles;
   g.ntiles = p.ntiles;
-  g.ksplit = std::max(1, ksplit);
-  const int grid = (p.ntiles * g.ksplit + 7) / 8 * 8 * p.mtiles;
-  static const hipError_t attr = [] {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_h16_gemm<false>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(kH16Lds));
-    return e != hipSuccess ? e
-                           : hipFuncSetAttribute(reinterpret_cast<const void *>(&k_h16_gemm<true>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(kH16Lds));
-  }();
-  hip_check(attr, "fp16-copy gemm LDS size");
-  if (g.ksplit > 1)
-    hipLaunchKernelGGL(k_h16_gemm<true>, dim3(grid), dim3(256), kH16Lds, s, g);
-  else
-    hipLaunchKernelGGL(k_h16_gemm<false>, dim3(grid), dim3(256), kH16Lds, s, g);
+  g.ksplit = p.ksplit;
+  g.nblocks = (N + kH16Pad - 1) / kH16Pad * (kH16Pad / 32);
+  switch (p.shape) {
+    case 0: h16_launch<H16A>(g, s); break;
+    case 1: h16_launch<H16B>(g, s); break;
+    case 2: h16_launch<H16C>(g, s); break;
+    default: h16_launch<H16D>(g, s); break;
+  }
   hip_check(hipGetLastError(), "q8 fp16-copy gemm launch");
   if (g.ksplit > 1) {
     const size_t count4 = size_t(M) * N / 4;

@@ -41,7 +41,7 @@ struct Tuning {
   int fuse_mlp = 1;          // QNN_FUSE_MLP: recorded INT4 SwiGLU + down as one launch
   int fuse_moe = 1;          // QNN_FUSE_MOE: one-token routed experts (and route) as one launch
   int q8_gemm_min_rows = 4;  // QNN_Q8_GEMM_MIN_ROWS: rows from which Q8_0 Linear takes the GEMM
-  int gemm_h16 = 128;        // QNN_GEMM_H16: rows from which Q8_0 Linear runs over a pre-expanded fp16 copy (0: never)
+  int gemm_h16 = 128;        // QNN_GEMM_H16: rows from which Q8_0 Linear always runs over a pre-expanded fp16 copy (0: never)
   int gguf_gemm_rows = 12;   // QNN_GGUF_GEMM_ROWS: the same for the other GGUF encodings (0: never)
   int gemm_max_rows = 0;     // QNN_GEMM_MAX_ROWS: rows per GEMM launch, at most (0: the 4 GiB fragment limit)
   int attn_wgs = 512;        // QNN_ATTN_WGS: cached-attention workgroup target
@@ -355,6 +355,7 @@ struct Q8GemmPlan {
   int mb = 1;  // 32-row blocks of C per wave
   int nw = 4;  // waves per workgroup (workgroup tile 32 * mb * nw rows)
   int m_pad = 0, k_pad = 0, ksteps = 0, mtiles = 0, ntiles = 0;
+  int shape = 0, ksplit = 1;  // h16_plan only
   size_t frag_bytes = 0, exp_bytes = 0;  // workspace: fp16 A fragments, per-row exponents
 };
 Q8GemmPlan q8_gemm_plan(int M, int K, int N);
@@ -367,13 +368,12 @@ void q8_rowexp_launch(const GGLayout &l, void *w, hipStream_t s);
 // `ew` is the weight's row exponents (a Q8_0 weight's own, at rowexp_off).
 size_t q8_h16_bytes(int rows, int cols);
 void q8_expand_h16_launch(const GGLayout &l, const void *w, void *out, hipStream_t s);
-Q8GemmPlan q8_h16_plan(int M, int K, int N);
-// ksplit > 1 (h16_ksplit: small grids) splits K over that many workgroups per
-// tile, their partial products in `part` (ksplit * M * N floats, N % 4 == 0),
-// summed in slice order by a second launch; ksplit 1 writes C directly.
-int h16_ksplit(const Q8GemmPlan &p, int N);
+Q8GemmPlan h16_plan(int M, int K, int N, bool split);
+// The plan's ksplit > 1 (with `split`: small grids) splits K over that many
+// workgroups per tile, their partial products in `part` (ksplit * M * N floats,
+// N % 4 == 0), summed in slice order by a second launch; 1 writes C directly.
 void q8_h16_gemm_launch(const Q8GemmPlan &p, const float *a, int M, int K, int N, const int *ew, const void *w16,
-                        void *frag, int *ea, float *c, hipStream_t s, int ksplit = 1, float *part = nullptr);
+                        void *frag, int *ea, float *c, hipStream_t s, float *part);
 // The fp16 copy of a weight of any other GGUF encoding (qnn_gguf.hip): its
 // row exponents (range_exp of the row's largest |value|, one int per row of
 // the copy's q8_h16_bytes rows), then the values RNE(v * 2^-e) in

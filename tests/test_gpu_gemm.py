@@ -91,6 +91,27 @@ def test_fp16_copy_output_edges(ctx, rng, tune, m, n):
     ctx.Recycle(src)
 
 
+@pytest.mark.parametrize("m,k,n", [(4, 1024, 1024), (33, 1088, 1056), (65, 4096, 257), (127, 2048, 1026), (129, 512, 4100),
+                                   (97, 8192, 128)])
+def test_fp16_copy_shapes(ctx, rng, tune, m, k, n):
+    """The GEMM's workgroup shapes (32, 64 and 128 rows; 128 and 192 columns), Q8_0 weights of 1 M elements and more
+    from four rows: the same bits as the decoding kernel.  Q4_K, where K is also sliced: within TOL."""
+    w, a = q8(rng, n, k), rng.standard_normal((m, k)).astype(np.float32)
+    tune("QNN_GEMM_H16", "0")
+    want = run_linear(ctx, w, a, n)
+    tune("QNN_GEMM_H16", "128")
+    h0 = ctx.status().gemm_h16
+    got = run_linear(ctx, w, a, n)
+    assert ctx.status().gemm_h16 - h0 == 1
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    if m < 12 or k % 256:
+        return
+    w4 = hip.gguf_quantize(ENC_Q4_K, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    got = run_linear(ctx, w4, a, n, enc=ENC_Q4_K)
+    for r in {0, 31, 32, 63, 64, m - 1} & set(range(m)):
+        assert normwise_rel_err(got[r], oracle.cpu_linear(w4, ENC_Q4_K, a[r], k, n)) <= TOL, r
+
+
 @pytest.mark.parametrize("enc", [ENC_Q8_0, ENC_Q4_K])
 def test_rows_in_several_gemm_launches(ctx, rng, tune, enc):
     """Rows beyond one launch's limit run as consecutive launches (the limit keeps the activation

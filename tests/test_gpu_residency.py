@@ -179,3 +179,33 @@ def test_upload_memory_block(small, rng):
     with pytest.raises(hip.EArgumentException):
         ctx.Upload(hip.MemoryBlock(v.view(np.uint16)[:100], (100,), hip.DT_BF16))
     ctx.Recycle(t)
+
+
+def test_few_rows_make_no_fp16_copy_by_eviction(small, tune):
+    """Fewer rows than QNN_GEMM_H16: the fp16 copy is made where it fits beside what is resident, and no weight is
+    evicted for it; the product then decodes the Q8_0 tiles, to the same bits."""
+    from quicknn_amd import hip
+
+    ctx = small
+    m, k, n = 8, 1024, 2048
+    rng = np.random.default_rng(9)
+    ws = [hip.MemoryBlock.gguf(hip.gguf_quantize(hip.WE_Q8_0, (rng.standard_normal(n * k) * 0.02).astype(np.float32)),
+                               n, k, hip.WE_Q8_0) for _ in range(3)]
+    a, y, x = ctx.UploadRaw(rng.standard_normal((m, k)).astype(np.float32)), ctx.NewTensor(m * n), ctx.NewTensor(k)
+    y1 = ctx.NewTensor(n)
+    for w in ws:  # three Q8_0 weights, 6.6 of 9 MiB: no room for a copy of 4 MiB
+        ctx.Linear(y1, x, w, None, None, 1, k, n)
+    ctx.Download(y1)
+    s0 = ctx.status()
+    got = []
+    for w in ws:
+        ctx.Linear(y, a, w, None, None, m, k, n)
+        got.append(ctx.Download(y).copy())
+    s1 = ctx.status()
+    assert s1.weight_evictions == s0.weight_evictions and s1.gemm_h16 == s0.gemm_h16
+    tune("QNN_GEMM_H16", "4")
+    ctx.Linear(y, a, ws[2], None, None, m, k, n)  # always: evicts
+    assert np.array_equal(ctx.Download(y).view(np.uint32), got[2].view(np.uint32))
+    assert ctx.status().weight_evictions > s1.weight_evictions and ctx.status().gemm_h16 == s1.gemm_h16 + 1
+    for t in (a, y, x, y1):
+        ctx.Recycle(t)
