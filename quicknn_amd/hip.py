@@ -245,6 +245,27 @@ def float_bits(v: float) -> int:
 _identity = itertools.count(1)
 
 
+def _address(a: np.ndarray) -> int:
+    """``a.ctypes.data``, which builds an interface object on each use (2.2 us, a third of an op's host time); through
+    the buffer protocol 0.6.  What that refuses (read-only, empty, strided arrays) takes the property."""
+    try:
+        return ctypes.addressof(ctypes.c_char.from_buffer(a))
+    except (TypeError, ValueError, BufferError):
+        return a.ctypes.data
+
+
+_int_arrays: dict = {}  # length -> ctypes array type
+
+
+def _ints(args):
+    """A C int array of ``args``, of one element at least."""
+    n = max(1, len(args))
+    t = _int_arrays.get(n)
+    if t is None:
+        t = _int_arrays[n] = ctypes.c_int * n
+    return t(*args)
+
+
 class MemoryBlock:
     """TMemoryBlock view of host weight storage (Common.pas:135-155).
 
@@ -264,7 +285,7 @@ class MemoryBlock:
         self.identity = identity if identity is not None else next(_identity)
 
     def desc(self) -> _Weight:
-        return _Weight(self.identity, self.data.ctypes.data, self.offset, self.size, self.shape[0],
+        return _Weight(self.identity, _address(self.data), self.offset, self.size, self.shape[0],
                        self.shape[1] if len(self.shape) > 1 else 1, self.dtype, self.encoding)
 
     @staticmethod
@@ -573,13 +594,11 @@ class GPUContext:
 
     def Kernel(self, op: int, n: int, dst: Tensor | None, a: Tensor | None, b: Tensor | None, c: Tensor | None,
                args) -> None:
-        arr = (ctypes.c_int * max(1, len(args)))(*args)
-        _raise(lib().qnn_kernel(self.h, op, n, _th(dst), _th(a), _th(b), _th(c), arr, len(args)))
+        _raise(lib().qnn_kernel(self.h, op, n, _th(dst), _th(a), _th(b), _th(c), _ints(args), len(args)))
 
     def KernelWeights(self, op: int, n: int, dst: Tensor, a: Tensor, b: MemoryBlock | None,
                       c: MemoryBlock | None, args) -> None:
-        arr = (ctypes.c_int * max(1, len(args)))(*args)
-        _raise(lib().qnn_kernel_weights(self.h, op, n, dst.handle, a.handle, _wd(b), _wd(c), arr, len(args)))
+        _raise(lib().qnn_kernel_weights(self.h, op, n, dst.handle, a.handle, _wd(b), _wd(c), _ints(args), len(args)))
 
     def CachedAttention(self, dst: Tensor, q: Tensor, cache: Tensor, query_rows: int, capacity: int, heads: int,
                         kv_heads: int, dim: int, position: int, window: int = 0, softcap: float = 0.0,
