@@ -30,9 +30,9 @@
 // V), which two waves per SIMD run under each other's products.  At dim 128
 // that takes tiles of 32 keys (221 registers; 64 keys take 343, one wave per
 // SIMD).  A KV head's keys are split over two workgroups per CU; k_attn_merge
-// joins the parts.  Infinities and NaNs among a workgroup's keys send its part
-// to a plain loop over its rows, since 0 times them would reach rows that do
-// not see the key.
+// joins the parts.  Infinities and NaNs among a workgroup's keys or query rows
+// send its part to a plain loop over its rows, since 0 times them would reach
+// rows that do not see the key, and NaN where the score is infinite.
 //
 // Measured (rotary, append and attention; 32 query heads on 8, dim 128), 128
 // rows over 4096 keys 453 -> 64 us (64-key tiles 67), over 16384 keys 1914 ->
@@ -79,16 +79,14 @@ __device__ __forceinline__ int plane_exp(uint32_t maxbits) {
   return maxbits ? max(range_exp(__uint_as_float(maxbits)), -110) : -110;
 }
 
-// Two fp16 planes of eight values times a power of two.  CHECKED: an infinity
-// or NaN is in hi alone (unchecked values are known to be finite).
-template <bool CHECKED>
+// Two fp16 planes of eight finite values times a power of two.
 __device__ __forceinline__ void planes8(const float (&x)[8], float scale, uint4 &ph, uint4 &pl) {
   float hi[8], lo[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const float s = x[i] * scale;
     hi[i] = float(_Float16(s));
-    lo[i] = !CHECKED || isfinite(hi[i]) ? s - hi[i] : 0.0f;
+    lo[i] = s - hi[i];
   }
   ph = make_uint4(pack_h2(hi[0], hi[1]), pack_h2(hi[2], hi[3]), pack_h2(hi[4], hi[5]), pack_h2(hi[6], hi[7]));
   pl = make_uint4(pack_h2(lo[0], lo[1]), pack_h2(lo[2], lo[3]), pack_h2(lo[4], lo[5]), pack_h2(lo[6], lo[7]));
@@ -104,9 +102,10 @@ __device__ __forceinline__ Rsrc rsrc(const void *base, size_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, int(uint32_t(min(bytes, size_t(0xFFFFFFFFu)))),
                                            0x00020000);
 }
-// Four floats (any 4-byte alignment); zeros past the end of the buffer.
-__device__ __forceinline__ float4 ld4(Rsrc r, uint32_t voff, uint32_t soff) {
-  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, int(voff), int(soff), 0);
+// Four floats (any 4-byte alignment); zeros past the end of the buffer.  The
+// whole offset is the lane's: a scalar offset need not take part in the check.
+__device__ __forceinline__ float4 ld4(Rsrc r, uint32_t off) {
+  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, int(off), 0, 0);
   return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
 }
 
@@ -160,6 +159,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   // ---- this lane's query row as B fragments: dims 16 ds + 8 h .. + 7
   half8 qh[T::DS], ql[T::DS];
   float qscale;  // score scale without the tile's exponent
+  bool qbad = false;  // an infinity or NaN in this wave's query rows: 0 times it would be in the planes' products
   {
     float qv[T::DS][8];
     const float *qr = a.q + (size_t(r) * a.heads + head) * a.dim;
@@ -181,15 +181,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         qv[ds][e] = v.x, qv[ds][e + 1] = v.y, qv[ds][e + 2] = v.z, qv[ds][e + 3] = v.w;
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) mx = abs_bits(qv[ds][e]) < kInfBits ? max(mx, abs_bits(qv[ds][e])) : mx;
+      for (int e = 0; e < 8; ++e) mx = max(mx, abs_bits(qv[ds][e]));
     }
+    qbad = __ballot(mx >= kInfBits) != 0;
     mx = max(mx, uint32_t(dev::xor_lanes_i<32>(int(mx))));
     const int e = plane_exp(mx);
     const float s = ldexpf(1.0f, -e);
 #pragma unroll
     for (int ds = 0; ds < T::DS; ++ds) {
       uint4 ph, pl;
-      planes8<true>(qv[ds], s, ph, pl);
+      planes8(qv[ds], s, ph, pl);
       qh[ds] = as_half8(ph);
       ql[ds] = as_half8(pl);
     }
@@ -199,9 +200,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   // ---- tile loads: unit u < UK is 4 keys x 8 dims of K, else 4 channels x 8 keys of V
   float4 raw[T::NU][8];
   auto unit_of = [&](int j) { return __builtin_amdgcn_readfirstlane((tid & ~63) + 256 * j) + lane; };
-  // Buffer loads: per unit one register of offset, the element rows in the
-  // scalar offset; dims past the last read zeros.  Keys outside the
-  // workgroup's range and channels past the last are zeroed after the load.
+  // Buffer loads: dims past the last and keys past the capacity read zeros or
+  // other elements of the head.  Keys outside the workgroup's range and
+  // channels past the last are zeroed after the load.
   const Rsrc krs = rsrc(kt, size_t(a.dim) * a.cap * 4), vrs = rsrc(vb, size_t(a.cap) * a.dim * 4);
   uint32_t uoff[T::NU];
 #pragma unroll
@@ -220,13 +221,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     for (int j = 0; j < T::NU; ++j) {
       const int u = unit_of(j);
       if (u >= 2 * T::UK) continue;  // whole waves
+      // (Opaque, or the eight rows' sums are kept in registers of their own.)
+      uint32_t at = uoff[j] + k0 * (u - lane < T::UK ? 1u : uint32_t(a.dim)) * 4u;
+      asm("" : "+v"(at));
       if (u - lane < T::UK) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) raw[j][e] = ld4(krs, uoff[j], (uint32_t(e) * uint32_t(a.cap) + k0) * 4u);
+        for (int e = 0; e < 8; ++e) raw[j][e] = ld4(krs, at + uint32_t(e) * uint32_t(a.cap) * 4u);
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          raw[j][e] = ld4(vrs, uoff[j], (k0 + 8u * (e >> 2) + (e & 3)) * uint32_t(a.dim) * 4u);
+        for (int e = 0; e < 8; ++e) raw[j][e] = ld4(vrs, at + (8u * (e >> 2) + (e & 3)) * uint32_t(a.dim) * 4u);
       }
     }
   };
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
         for (int e = 0; e < 8; ++e)
           v[e] = i == 0 ? raw[j][e].x : (i == 1 ? raw[j][e].y : (i == 2 ? raw[j][e].z : raw[j][e].w));
-        planes8<false>(v, s, dst[i], dst[plane + i]);
+        planes8(v, s, dst[i], dst[plane + i]);
       }
     }
   };
@@ -329,14 +332,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       uint32_t mk, mv;
       wave_max(mk, mv);
       if (lane == 0) {
-        red[par][0][wave] = mk;
+        red[par][0][wave] = qbad ? kInfBits : mk;
         red[par][1][wave] = mv;
       }
     }
     __syncthreads();  // the maxima, and every wave is done with the previous tile's fragments
     uint32_t mk = max(max(red[par][0][0], red[par][0][1]), max(red[par][0][2], red[par][0][3]));
     uint32_t mv = max(max(red[par][1][0], red[par][1][1]), max(red[par][1][2], red[par][1][3]));
-    if (mk >= kInfBits || mv >= kInfBits) {  // uniform: an infinity or NaN among the keys
+    if (mk >= kInfBits || mv >= kInfBits) {  // uniform: an infinity or NaN among the keys or in q
       slow = true;
       break;
     }
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
         for (int e = 0; e < 8; ++e) pv[e] = s[ks >> 1][8 * (ks & 1) + e];
         uint4 ph, pl;
-        planes8<false>(pv, 16384.0f, ph, pl);
+        planes8(pv, 16384.0f, ph, pl);
         p_h[ks & 1] = as_half8(ph);
         p_l[ks & 1] = as_half8(pl);
       };
@@ -455,8 +458,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   }
   if (slow) {
     // Infinities or NaNs among the keys would reach rows that do not see them
-    // through the products' zeros: this part is computed row by row instead, a
-    // wave per query row, in fp32 as k_attn does.
+    // through the products' zeros, and in q would meet the zeros of the lower
+    // planes (inf, which a soft cap makes finite, would be NaN): this part is
+    // computed row by row instead, a wave per query row, in fp32 as k_attn does.
     for (int i = wave; i < kQRows && q0 + i < nq; i += 4) {
       const int row = (q0 + i) / a.group, hd = kh * a.group + (q0 + i) % a.group;
       const float *qr = a.q + (size_t(row) * a.heads + hd) * a.dim;
@@ -471,7 +475,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         float sc = dev::wave_sum_xor(d) * mul;
         if (a.softcap > 0.0f) sc = a.softcap * tanhf(fminf(fmaxf(sc / a.softcap, -20.0f), 20.0f));
         const float mn = fmaxf(m, sc);
-        const float kp = mn == -INFINITY ? 1.0f : expf(m - mn), w = mn > -INFINITY ? expf(sc - mn) : 0.0f;
+        // (a NaN before any other key counts, too)
+        const float kp = mn == -INFINITY ? 1.0f : expf(m - mn), w = sc == -INFINITY ? 0.0f : expf(sc - mn);
         l = l * kp + w;
         m = mn;
         for (int c = lane, j = 0; c < a.dim; c += 64, ++j) {

@@ -208,10 +208,10 @@ __global__ __launch_bounds__(512) void k_i4_gemm(const I4GemmArgs a) {
     const uint32_t st = lds0 + uint32_t(kt % SG::ST) * SG::BYTES, ktg = uint32_t(kt0 + kt);
     if (i < SG::APW)
       gemm_dma16(dev::rsrc(a.frag, live ? abytes : 0u), __builtin_amdgcn_readfirstlane(st + uint32_t(ap + i) * 1024u),
-                 l16, asoff + ktg * 8192u + uint32_t(i) * 1024u);
+                 l16, live ? asoff + ktg * 8192u + uint32_t(i) * 1024u : 0u);
     else
       gemm_dma16(dev::rsrc(lbase, live ? lsize : 0u), __builtin_amdgcn_readfirstlane(st + ldst), l16,
-                 ((2u * ktg + uint32_t(lg)) >> lshift) * 1024u);
+                 live ? ((2u * ktg + uint32_t(lg)) >> lshift) * 1024u : 0u);
   };
 #pragma unroll
   for (int k = 0; k < SG::ST - 1; ++k)

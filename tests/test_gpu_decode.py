@@ -396,6 +396,31 @@ def test_attention_of_many_rows_infinite_keys(ctx, rng, tune, where, value):
         ctx.Recycle(z)
 
 
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_attention_of_many_rows_infinite_queries(ctx, rng, tune, value, softcap):
+    """An infinity or NaN in a query row gives what k_attn gives (with a soft cap an infinite score is a finite one);
+    the capacity ends in the middle of a tile, and what follows the cache in its tensor is not read."""
+    case = (48, 8, 2, 128, 149, 101, 0, softcap, 0.0, False)
+    rows, heads, kvh, dim, cap, pos, window, softcap, scale, masked = case
+    q, cache = many_inputs(rng, case)
+    q.reshape(rows, heads, dim)[20, 3, 7] = value
+    q.reshape(rows, heads, dim)[47, 7, 0] = value
+    cache = np.concatenate([cache, np.full(64 * 128, np.nan, np.float32)])
+    tq, tc, to = up(ctx, q), up(ctx, cache), ctx.NewTensor(rows * heads * dim)
+    got = {}
+    for mm in ("1", "0"):
+        tune("QNN_ATTN_MM", mm)
+        ctx.CachedAttention(to, tq, tc, rows, cap, heads, kvh, dim, pos, window, softcap, scale, masked)
+        got[mm] = ctx.Download(to).reshape(rows, heads, dim)
+    a, b = got["1"], got["0"]
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.all(np.isfinite(np.delete(b, (20, 47), axis=0)))
+    fine = ~np.isnan(b)
+    assert np.max(np.abs(a[fine] - b[fine])) <= 1e-5 * np.max(np.abs(b[fine]))
+    for z in (tq, tc, to):
+        ctx.Recycle(z)
+
+
 @pytest.mark.parametrize("vocab,k,levels", [
     (1, 1, 0), (63, 64, 0), (4095, 64, 0), (4097, 40, 3), (8192, 3, 0), (9000, 64, 1), (20000, 64, 1), (20000, 33, 40),
     (263000, 64, 0), (263000, 64, 2)])
