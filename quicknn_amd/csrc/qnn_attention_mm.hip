@@ -43,7 +43,13 @@
 // From when (attn_mm_plan): four rows, and rows x heads x keys of 512 k: 4
 // rows of 32 heads over 4096 keys 32.2 -> 31.0 us, 2 rows 27.1 -> 30.6 (over
 // 16384 keys 49.3 -> 63.2); 32 rows of 16 heads over 512 keys 26.6 -> 31.0,
-// 128 rows 43.9 -> 34.6.
+// 128 rows 43.9 -> 34.6.  With 65 to 96 channels, one workgroup per CU, 640 k:
+// 58 rows of 8 heads on 4, dim 80, soft cap, over 1207 keys (547 k) 33.3 ->
+// 37.3; 107 rows of 8 on 2 over 1097 (917 k) 37.9 -> 28.9.
+// Soft cap: tanhf and a division by the cap took as long as all else on the
+// VALU; tanh20 and a product: 20 rows of 28 heads on 4 over 2794 keys 40.3 ->
+// 36.5 us, 102 rows of 8 on 4 over 765 keys, dim 64, 32.4 -> 28.4 (k_attn:
+// 213.6, 32.2); error against 64 bits 3.34e-7 -> 3.38e-7.
 #include "qnn_internal.h"
 #include "qnn_lanes.h"
 
@@ -95,6 +101,20 @@ __device__ __forceinline__ half8 as_half8(const uint4 &v) {
   half8 h;
   __builtin_memcpy(&h, &v, 16);
   return h;
+}
+
+// tanh for |x| <= 20: below 0.6 x + x^3 P(x^2), P fitted by least squares at
+// Chebyshev nodes (4e-9 relative), above 1 - 2 / (e^2|x| + 1).  Within 1.7e-7
+// of the value, as tanhf is (2 ulp), in 14 operations and no branch.
+__device__ __forceinline__ float tanh20(float x) {
+  const float a = fabsf(x), z = x * x;
+  float p = fmaf(-0.00597367529f, z, 0.0208660811f);
+  p = fmaf(p, z, -0.053805545f);
+  p = fmaf(p, z, 0.133321926f);
+  p = fmaf(p, z, -0.333333075f);
+  const float small = fmaf(a * z, p, a);
+  const float large = fmaf(-2.0f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a * 2.88539008f) + 1.0f), 1.0f);
+  return copysignf(a < 0.6f ? small : large, x);
 }
 
 typedef __amdgpu_buffer_rsrc_t Rsrc;
@@ -376,11 +396,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         __builtin_amdgcn_sched_barrier(0);
       }
       if (EXTRA && a.softcap > 0.0f) {
+        const float inv = 1.0f / a.softcap;
 #pragma unroll
         for (int kb = 0; kb < T::KB; ++kb)
 #pragma unroll
           for (int i = 0; i < 16; ++i)
-            s[kb][i] = a.softcap * tanhf(fminf(fmaxf(s[kb][i] / a.softcap, -20.0f), 20.0f));
+            s[kb][i] = a.softcap * tanh20(fminf(fmaxf(s[kb][i] * inv, -20.0f), 20.0f));
       }
       const int k0 = t * KT;
       const bool valid_all = k0 >= both0 && k0 + KT <= both1 && !(EXTRA && a.masked);  // uniform
@@ -552,9 +573,10 @@ bool attn_mm_plan(AttnPlan &p, int rows, int cap, int heads, int kv_heads, int d
   const int group = heads / kv_heads, min_k = tuning().attn_mm_min;
   const long long nq = (long long)rows * group;
   const int last_end = position + rows;
+  const long long least = ((long long)min_k << 10) * (dim > 64 && dim <= 96 ? 5 : 4) / 4;
   if (min_k <= 0 || rows < 4 || dim > 128 || nq > (1 << 24) ||
       size_t(dim) * cap * 4 > 0x7FFFFFFFull ||  // 32-bit offsets within a KV head
-      (long long)rows * heads * (window > 0 ? std::min(window, last_end) : last_end) < (long long)min_k << 10)
+      (long long)rows * heads * (window > 0 ? std::min(window, last_end) : last_end) < least)
     return false;
   p.qtiles = int((nq + kQRows - 1) / kQRows);
   // The keys of one workgroup's rows: at most the window and those rows.

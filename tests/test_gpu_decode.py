@@ -319,6 +319,8 @@ MANY = [
     (50, 16, 2, 96, 400, 333, 100, 0.0, 0.05, False),  # window, scale
     (24, 8, 2, 128, 300, 200, 31, 30.0, 0.0, True),   # window shorter than a tile, soft cap, mask
     (64, 4, 1, 64, 200, 100, 0, 20.0, 0.0, True),
+    (36, 8, 2, 64, 200, 100, 0, 2.0, 0.0, False),     # soft cap: scores on both sides of 0.6 of it, and far above
+    (30, 8, 2, 80, 200, 100, 0, 50.0, 0.0, False),    # scores far below it
 ]
 
 
