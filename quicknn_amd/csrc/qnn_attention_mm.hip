@@ -8,12 +8,17 @@
 // walks a range of keys once, in tiles of KT.
 //
 // Both products take fp32 operands as two fp16 planes, hi = fp16(v), lo =
-// fp16(v - hi), 22 significant bits, and run hi hi + lo hi + hi lo on
-// v_mfma_f32_32x32x16_f16 with fp32 accumulation; scores, softmax, running
-// maxima and sums are fp32.  Powers of two keep the planes in fp16's range: q
-// per row, K per tile, V by the largest of the tiles so far, p by 2^14 (each
-// plane then resolves 2^-38 of the largest value it is scaled for).  The error
-// against 64 bits is no larger than that of k_attn's fp32 sums.
+// fp16(v - hi), and run hi hi + lo hi + hi lo on v_mfma_f32_32x32x16_f16 with
+// fp32 accumulation; scores, softmax, running maxima and sums are fp32.  hi and
+// lo hold a value to 2^-24 of itself, as long as lo is a normal fp16 number:
+// down to 2^-15 or so of the largest that shares its scale, below that to 2^-38
+// of that largest.  So what has a scale of its own is small: every key's K and
+// V (a score is one key's, and a key's V scale goes into its weight), every
+// query row, and every row's weights w = p 2^(V's exponent), by the largest w
+// of the row so far.  A key that a row does not see, by the mask, a later
+// position or the window, has w = 0 there, and whatever finite values it holds
+// reach nothing else; with one scale for a tile's keys a hidden value of 1e8
+// times the others cost the result 1e-4, of 1e12 all of it.
 //
 // Layout.  S^T = K Q^T, so a lane's results are keys of ONE query row (column
 // l % 32): maxima and sums are in-lane but for one exchange of the two
@@ -28,28 +33,30 @@
 // What bounds it: per 64 keys and wave 96 MFMAs (18.5 ns each) against about
 // 1000 VALU operations (softmax, planes of p, a share of the planes of K and
 // V), which two waves per SIMD run under each other's products.  At dim 128
-// that takes tiles of 32 keys (221 registers; 64 keys take 343, one wave per
+// that takes tiles of 32 keys (236 registers; 64 keys do not fit two waves per
 // SIMD).  A KV head's keys are split over two workgroups per CU; k_attn_merge
 // joins the parts.  Infinities and NaNs among a workgroup's keys or query rows
 // send its part to a plain loop over its rows, since 0 times them would reach
 // rows that do not see the key, and NaN where the score is infinite.
+// More than 128 channels stay with k_attn: at 256 the output of 32 rows (128
+// registers) and the planes of q (128) are all that a wave of two per SIMD has.
 //
 // Measured (rotary, append and attention; 32 query heads on 8, dim 128), 128
-// rows over 4096 keys 453 -> 64 us (64-key tiles 67), over 16384 keys 1914 ->
-// 159 (190), 64 rows 232 -> 48, 16 rows 73 -> 33, 8 rows 45 -> 30 us; error
-// against 64 bits 5.9e-7 -> 3.9e-7.  One against two workgroups per CU: 69
-// against 64 us, 191 against 159; with four, 77 and 172.  At dim 96, where one
-// fits a CU, 128 rows of 16 heads on 8 over 3000 keys: one 41, two 46 us.
+// rows over 4096 keys 453 -> 63 us, over 16384 keys 1900 -> 160, 64 rows 224 ->
+// 48, 16 rows 72 -> 31, 8 rows 45 -> 30 us (scales per tile and not per key: 1 to
+// 3 us less, all in the two larger).  One against two workgroups per CU: 69
+// against 65 us, 192 against 160; with four, 77 and 170.  Error against 64 bits
+// 5.9e-7 -> 3.4e-7; over 60 drawn shapes that come here 0.74 to 0.84 of k_attn's.
 // From when (attn_mm_plan): four rows, and rows x heads x keys of 512 k: 4
-// rows of 32 heads over 4096 keys 32.2 -> 31.0 us, 2 rows 27.1 -> 30.6 (over
-// 16384 keys 49.3 -> 63.2); 32 rows of 16 heads over 512 keys 26.6 -> 31.0,
-// 128 rows 43.9 -> 34.6.  With 65 to 96 channels, one workgroup per CU, 640 k:
-// 58 rows of 8 heads on 4, dim 80, soft cap, over 1207 keys (547 k) 33.3 ->
-// 37.3; 107 rows of 8 on 2 over 1097 (917 k) 37.9 -> 28.9.
+// rows of 32 heads over 4096 keys 31.2 -> 29.1 us, 2 rows 27.1 -> 30.6 (over
+// 16384 keys 49.3 -> 63.2); 32 rows of 16 heads over 512 keys 26.0 -> 29.9,
+// 128 rows 41.2 -> 32.9.  With 65 to 96 channels 640 k: 58 rows of 8 heads on
+// 4, dim 80, soft cap, over 1207 keys (547 k) 32.6 -> 36.9; 107 rows of 8 on 2
+// over 1097 (917 k) 39.3 -> 30.6.
 // Soft cap: tanhf and a division by the cap took as long as all else on the
 // VALU; tanh20 and a product: 20 rows of 28 heads on 4 over 2794 keys 40.3 ->
-// 36.5 us, 102 rows of 8 on 4 over 765 keys, dim 64, 32.4 -> 28.4 (k_attn:
-// 213.6, 32.2); error against 64 bits 3.34e-7 -> 3.38e-7.
+// 36.5 us, 102 rows of 8 on 4 over 765 keys, dim 64, 32.4 -> 28.4; error against
+// 64 bits 3.34e-7 -> 3.38e-7.
 #include "qnn_internal.h"
 #include "qnn_lanes.h"
 
@@ -60,7 +67,6 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kQRows = 128;  // query rows (of one KV head) per workgroup, 32 per wave
-constexpr int kPExp = 14;    // p is held as p 2^14
 constexpr uint32_t kInfBits = 0x7F800000u;
 
 struct AttnMmArgs {
@@ -71,32 +77,76 @@ struct AttnMmArgs {
 };
 
 __device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFu; }
-__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
-  v = max(v, uint32_t(dev::xor_lanes_i<32>(int(v))));
-  v = max(v, uint32_t(dev::xor_lanes_i<16>(int(v))));
-  v = max(v, uint32_t(dev::xor_lanes_i<8>(int(v))));
-  v = max(v, uint32_t(dev::xor_lanes_i<4>(int(v))));
-  v = max(v, uint32_t(dev::xor_lanes_i<2>(int(v))));
-  return max(v, uint32_t(dev::xor_lanes_i<1>(int(v))));
-}
-// Exponent for a largest finite magnitude; below 2^-110 (and for zeros, which
-// ask for none) the scale stays 2^110, which is finite.
-__device__ __forceinline__ int plane_exp(uint32_t maxbits) {
-  return maxbits ? max(range_exp(__uint_as_float(maxbits)), -110) : -110;
-}
+// A power of two for the planes of a row or key from its largest magnitude's
+// bits: its exponent field, 2^-112 at least.  plane_scale brings the magnitude
+// into [2^14, 2^15); plane_exp is the exponent that undoes it.
+__device__ __forceinline__ uint32_t exp_field(uint32_t maxbits) { return max(maxbits & kInfBits, 15u << 23); }
+__device__ __forceinline__ float plane_scale(uint32_t field) { return __uint_as_float((268u << 23) - field); }
+__device__ __forceinline__ int plane_exp(uint32_t field) { return int(field >> 23) - 141; }
 
-// Two fp16 planes of eight finite values times a power of two.
-__device__ __forceinline__ void planes8(const float (&x)[8], float scale, uint4 &ph, uint4 &pl) {
+// Two fp16 planes of eight finite values, each times its power of two.
+__device__ __forceinline__ void planes8(const float (&x)[8], const float (&scale)[8], uint4 &ph, uint4 &pl) {
   float hi[8], lo[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float s = x[i] * scale;
+    const float s = x[i] * scale[i];
     hi[i] = float(_Float16(s));
     lo[i] = s - hi[i];
   }
   ph = make_uint4(pack_h2(hi[0], hi[1]), pack_h2(hi[2], hi[3]), pack_h2(hi[4], hi[5]), pack_h2(hi[6], hi[7]));
   pl = make_uint4(pack_h2(lo[0], lo[1]), pack_h2(lo[2], lo[3]), pack_h2(lo[4], lo[5]), pack_h2(lo[6], lo[7]));
 }
+__device__ __forceinline__ void planes8(const float (&x)[8], float scale, uint4 &ph, uint4 &pl) {
+  const float s[8] = {scale, scale, scale, scale, scale, scale, scale, scale};
+  planes8(x, s, ph, pl);
+}
+
+// Largest values over pairs of lanes, sixteen or thirty-two apart, of two
+// values at once: lanes with that bit clear get a's, the others b's.
+__device__ __forceinline__ uint32_t max_halves(uint32_t a, uint32_t b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  return max(uint32_t(r[0]), uint32_t(r[1]));
+}
+__device__ __forceinline__ uint32_t max_rows(uint32_t a, uint32_t b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  return max(uint32_t(r[0]), uint32_t(r[1]));
+}
+// The same for lanes one or two apart.
+template <int OFF>
+__device__ __forceinline__ uint32_t max_near(uint32_t a, uint32_t b, bool upper) {
+  return max(upper ? b : a, uint32_t(dev::xor_lanes_i<OFF>(int(upper ? a : b))));
+}
+// A key's largest magnitude of K: m of a lane's four keys over the lanes that
+// hold its other dims (bits 4 and 5, with tiles of 32 keys 3 too).  The lane
+// keeps key lane / 16.
+template <int KT>
+__device__ __forceinline__ uint32_t k_key_max(const uint32_t (&m)[4]) {
+  uint32_t v = max_rows(max_halves(m[0], m[2]), max_halves(m[1], m[3]));
+  if (KT == 32) v = max(v, uint32_t(dev::xor_lanes_i<8>(int(v))));
+  return v;
+}
+// A key's largest magnitude of V: m of a lane's eight keys over the lanes that
+// hold its other channels: bits 0-2 and 5, with tiles of 32 keys 4 too.  The
+// lane keeps key v_kept.
+template <int KT>
+__device__ __forceinline__ uint32_t v_key_max(const uint32_t (&m)[8], int lane) {
+  constexpr int N = KT == 32 ? 2 : 4;
+  uint32_t v[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    v[i] = KT == 32 ? max_rows(max_halves(m[i], m[4 + i]), max_halves(m[2 + i], m[6 + i])) : max_halves(m[i], m[4 + i]);
+    v[i] = max(v[i], uint32_t(__builtin_amdgcn_mov_dpp(int(v[i]), 0x141, 0xF, 0xF, false)));  // lane 7 - l of its eight
+  }
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) v[i] = max_near<1>(v[2 * i], v[2 * i + 1], lane & 1);
+  if (KT == 32) return max(v[0], uint32_t(dev::xor_lanes_i<2>(int(v[0]))));
+  return max_near<2>(v[0], v[1], lane & 2);
+}
+template <int KT>
+__device__ __forceinline__ int v_kept(int lane) {
+  return (lane & 1) + (KT == 32 ? lane >> 3 & 2 : lane & 2) + (lane >> 3 & 4);
+}
+
 __device__ __forceinline__ half8 as_half8(const uint4 &v) {
   half8 h;
   __builtin_memcpy(&h, &v, 16);
@@ -129,15 +179,23 @@ __device__ __forceinline__ float4 ld4(Rsrc r, uint32_t off) {
   return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
 }
 
-// DP: head dimension padded to a multiple of 32; KT: keys per tile.
+// DP: head dimension padded to a multiple of 32; KT: keys per tile.  Waves 0
+// and 1 hold a tile's K, thread x of them 4 keys from 4 (x % (KT / 4)) by 8 dims
+// from 8 (x / (KT / 4)); waves 2 and 3 its V, thread x 8 keys by 4 channels.
 template <int DP, int KT>
 struct AttnMm {
   static constexpr int DS = DP / 16, CB = DP / 32, KB = KT / 32, KS = KT / 16;
-  static constexpr int UK = KT * DP / 32;            // units of 4 x 8 elements of K, and as many of V
-  static constexpr int NU = (2 * UK + 255) / 256;    // per thread
   static constexpr int KF = KB * DS * 64, VF = CB * KS * 64;  // 16-byte pieces per plane
   static constexpr size_t lds = size_t(2 * KF + 2 * VF) * 16;
-  static_assert(UK % 64 == 0, "whole waves take K or V units");
+  static constexpr bool SPARE = KT * DP < 32 * 128;  // the last threads of both have dims, channels past DP
+  static_assert(KT * DP <= 32 * 128, "a tile is 128 threads of 4 x 8 elements");
+  // V: the channels from 4 v_group, the keys 16 (kk / 2) + 4 (kk % 2) + 0..3 and
+  // 8..11.  Eight lanes read 128 bytes of a key; what else of a key the wave
+  // holds lies in upper lanes (v_key_max).
+  static __device__ __forceinline__ int v_group(int x) { return (x & 7) + (KT == 32 ? x >> 1 & 24 : x >> 2 & 8); }
+  static __device__ __forceinline__ int v_kk(int x) {
+    return KT == 32 ? (x >> 3 & 1) + (x >> 5 & 2) : (x >> 3 & 3) + (x >> 4 & 4);
+  }
 };
 
 // EXTRA: a key mask or a soft cap.
@@ -146,7 +204,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   using T = AttnMm<DP, KT>;
   extern __shared__ uint4 lds[];
   uint4 *kf = lds, *vf = lds + 2 * T::KF;  // [plane][key block][dim step][lane], [plane][channel block][key step][lane]
-  __shared__ uint32_t red[2][2][4];        // [tile parity][K, V][wave]
+  __shared__ __align__(16) uint32_t kmx[2][KT], vmx[KT];  // the tile's keys' largest magnitudes of K (per wave), V
+  __shared__ __align__(16) int kex[KT];                   // exponents of their K planes
+  __shared__ __align__(16) float vpw[KT];                 // powers of two of their V
+  __shared__ __align__(16) uint32_t bad[4];               // per wave: an infinity or NaN
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int p = lane & 31, h = lane >> 5;
   // KV head fastest: with eight of them each XCD (as workgroups are usually
@@ -178,10 +239,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
   // ---- this lane's query row as B fragments: dims 16 ds + 8 h .. + 7
   half8 qh[T::DS], ql[T::DS];
-  float qscale;  // score scale without the tile's exponent
+  int qexp;  // exponent of a score, but for the key's
   bool qbad = false;  // an infinity or NaN in this wave's query rows: 0 times it would be in the planes' products
   {
     float qv[T::DS][8];
+    // The score's scale as a factor in [0.5, 1), taken into q, and an exponent.
+    int sexp;
+    const float sfac = frexpf(a.scale > 0.0f ? a.scale : 1.0f / sqrtf(float(a.dim)), &sexp);
     const float *qr = a.q + (size_t(r) * a.heads + head) * a.dim;
     uint32_t mx = 0;
 #pragma unroll
@@ -201,12 +265,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         qv[ds][e] = v.x, qv[ds][e + 1] = v.y, qv[ds][e + 2] = v.z, qv[ds][e + 3] = v.w;
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) mx = max(mx, abs_bits(qv[ds][e]));
+      for (int e = 0; e < 8; ++e) {
+        qv[ds][e] *= sfac;
+        mx = max(mx, abs_bits(qv[ds][e]));
+      }
     }
     qbad = __ballot(mx >= kInfBits) != 0;
     mx = max(mx, uint32_t(dev::xor_lanes_i<32>(int(mx))));
-    const int e = plane_exp(mx);
-    const float s = ldexpf(1.0f, -e);
+    const uint32_t ef = exp_field(mx);
+    const float s = plane_scale(ef);
 #pragma unroll
     for (int ds = 0; ds < T::DS; ++ds) {
       uint4 ph, pl;
@@ -214,124 +281,128 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       qh[ds] = as_half8(ph);
       ql[ds] = as_half8(pl);
     }
-    qscale = ldexpf(a.scale > 0.0f ? a.scale : 1.0f / sqrtf(float(a.dim)), e);
+    qexp = plane_exp(ef) + sexp;
   }
 
-  // ---- tile loads: unit u < UK is 4 keys x 8 dims of K, else 4 channels x 8 keys of V
-  float4 raw[T::NU][8];
-  auto unit_of = [&](int j) { return __builtin_amdgcn_readfirstlane((tid & ~63) + 256 * j) + lane; };
+  // ---- this thread's share of a tile
+  float4 raw[8];  // K: dim e of the four keys; V: key e's four channels
+  const bool isk = wave < 2;  // uniform
+  const int x = tid & 127;
+  const int kkey = 4 * (x % (KT / 4)), kdim = 8 * (x / (KT / 4));
+  const int vch = 4 * T::v_group(x), vkey = 16 * (T::v_kk(x) >> 1) + 4 * (T::v_kk(x) & 1);
+  const bool spare = T::SPARE && (isk ? kdim : vch) >= DP;  // nothing to hold, whatever was loaded
   // Buffer loads: dims past the last and keys past the capacity read zeros or
   // other elements of the head.  Keys outside the workgroup's range and
   // channels past the last are zeroed after the load.
   const Rsrc krs = rsrc(kt, size_t(a.dim) * a.cap * 4), vrs = rsrc(vb, size_t(a.cap) * a.dim * 4);
-  uint32_t uoff[T::NU];
-#pragma unroll
-  for (int j = 0; j < T::NU; ++j) {
-    const int u = unit_of(j);
-    if (u - lane < T::UK) {
-      uoff[j] = (uint32_t(8 * (u / (KT / 4))) * uint32_t(a.cap) + uint32_t(4 * (u % (KT / 4)))) * 4u;
-    } else {
-      const int x = u - T::UK, kk = x / (DP / 4);
-      uoff[j] = (uint32_t(16 * (kk >> 1) + 4 * (kk & 1)) * uint32_t(a.dim) + uint32_t(4 * (x % (DP / 4)))) * 4u;
-    }
-  }
+  const uint32_t off0 = (isk ? uint32_t(kdim) * uint32_t(a.cap) + uint32_t(kkey) : uint32_t(vkey) * uint32_t(a.dim) + uint32_t(vch)) * 4u;
   auto load_tile = [&](int t) {
-    const uint32_t k0 = uint32_t(t) * KT;
+    // (Opaque, or the eight rows' sums are kept in registers of their own.)
+    uint32_t at = off0 + uint32_t(t) * KT * (isk ? 1u : uint32_t(a.dim)) * 4u;
+    asm("" : "+v"(at));
+    if (isk) {
 #pragma unroll
-    for (int j = 0; j < T::NU; ++j) {
-      const int u = unit_of(j);
-      if (u >= 2 * T::UK) continue;  // whole waves
-      // (Opaque, or the eight rows' sums are kept in registers of their own.)
-      uint32_t at = uoff[j] + k0 * (u - lane < T::UK ? 1u : uint32_t(a.dim)) * 4u;
-      asm("" : "+v"(at));
-      if (u - lane < T::UK) {
+      for (int e = 0; e < 8; ++e) raw[e] = ld4(krs, at + uint32_t(e) * uint32_t(a.cap) * 4u);
+    } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) raw[j][e] = ld4(krs, at + uint32_t(e) * uint32_t(a.cap) * 4u);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) raw[j][e] = ld4(vrs, at + (8u * (e >> 2) + (e & 3)) * uint32_t(a.dim) * 4u);
-      }
+      for (int e = 0; e < 8; ++e) raw[e] = ld4(vrs, at + (8u * (e >> 2) + (e & 3)) * uint32_t(a.dim) * 4u);
     }
   };
   auto trim_tile = [&](int t) {
     const int k0 = t * KT;
     const bool inside = k0 >= klo && k0 + KT <= khi;  // uniform
     if (inside && a.dim == DP) return;
+    if (isk) {
+      const int key = k0 + kkey;
+      if (inside) return;
 #pragma unroll
-    for (int j = 0; j < T::NU; ++j) {
-      const int u = unit_of(j);
-      if (u >= 2 * T::UK) continue;
-      if (u - lane < T::UK) {
-        const int key = k0 + 4 * (u % (KT / 4));
-        if (inside) continue;
+      for (int e = 0; e < 8; ++e) {
+        float4 &v = raw[e];
+        v.x = key >= klo && key < khi ? v.x : 0.0f;
+        v.y = key + 1 >= klo && key + 1 < khi ? v.y : 0.0f;
+        v.z = key + 2 >= klo && key + 2 < khi ? v.z : 0.0f;
+        v.w = key + 3 >= klo && key + 3 < khi ? v.w : 0.0f;
+      }
+    } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          float4 &v = raw[j][e];
-          v.x = key >= klo && key < khi ? v.x : 0.0f;
-          v.y = key + 1 >= klo && key + 1 < khi ? v.y : 0.0f;
-          v.z = key + 2 >= klo && key + 2 < khi ? v.z : 0.0f;
-          v.w = key + 3 >= klo && key + 3 < khi ? v.w : 0.0f;
-        }
-      } else {
-        const int x = u - T::UK, ch = 4 * (x % (DP / 4)), kk = x / (DP / 4);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = k0 + 16 * (kk >> 1) + 8 * (e >> 2) + 4 * (kk & 1) + (e & 3);
-          const int n = key >= klo && key < khi ? a.dim - ch : 0;  // channels from ch
-          float4 &v = raw[j][e];
-          v.x = n > 0 ? v.x : 0.0f;
-          v.y = n > 1 ? v.y : 0.0f;
-          v.z = n > 2 ? v.z : 0.0f;
-          v.w = n > 3 ? v.w : 0.0f;
-        }
+      for (int e = 0; e < 8; ++e) {
+        const int key = k0 + vkey + 8 * (e >> 2) + (e & 3);
+        const int n = key >= klo && key < khi ? a.dim - vch : 0;  // channels from vch
+        float4 &v = raw[e];
+        v.x = n > 0 ? v.x : 0.0f;
+        v.y = n > 1 ? v.y : 0.0f;
+        v.z = n > 2 ? v.z : 0.0f;
+        v.w = n > 3 ? v.w : 0.0f;
       }
     }
   };
-  // Largest magnitude bits of this wave's K units and V units.
-  auto wave_max = [&](uint32_t &mk, uint32_t &mv) {
-    mk = mv = 0;
+  // Every key's largest magnitudes, of K as far as this wave holds it.
+  auto key_maxima = [&]() {
+    uint32_t top;
+    if (isk) {
+      uint32_t m[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int j = 0; j < T::NU; ++j) {
-      const int u = unit_of(j);
-      if (u >= 2 * T::UK) continue;
-      uint32_t m = 0;
+      for (int e = 0; e < 8; ++e) {
+        m[0] = max(m[0], abs_bits(raw[e].x));
+        m[1] = max(m[1], abs_bits(raw[e].y));
+        m[2] = max(m[2], abs_bits(raw[e].z));
+        m[3] = max(m[3], abs_bits(raw[e].w));
+      }
+      top = k_key_max<KT>(m);
+      kmx[wave & 1][kkey + (lane >> 4)] = top;
+    } else {
+      uint32_t m[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        m = max(max(max(m, abs_bits(raw[j][e].x)), abs_bits(raw[j][e].y)),
-                max(abs_bits(raw[j][e].z), abs_bits(raw[j][e].w)));
-      if (u - lane < T::UK) mk = max(mk, m);
-      else mv = max(mv, m);
+      for (int e = 0; e < 8; ++e) {
+        m[e] = max(max(abs_bits(raw[e].x), abs_bits(raw[e].y)), max(abs_bits(raw[e].z), abs_bits(raw[e].w)));
+        if (spare) m[e] = 0u;
+      }
+      top = v_key_max<KT>(m, lane);
+      const int e = v_kept<KT>(lane);
+      vmx[vkey + 8 * (e >> 2) + (e & 3)] = top;
     }
-    mk = wave_umax(mk);
-    mv = wave_umax(mv);
+    const bool inf = qbad || __ballot(top >= kInfBits) != 0;
+    if (lane == 0) bad[wave] = inf;
   };
-  auto write_tile = [&](float ks, float vs) {
+  auto k_field4 = [&](int key) {
+    const uint4 m = *reinterpret_cast<const uint4 *>(&kmx[0][key]), o = *reinterpret_cast<const uint4 *>(&kmx[1][key]);
+    return make_uint4(exp_field(max(m.x, o.x)), exp_field(max(m.y, o.y)), exp_field(max(m.z, o.z)), exp_field(max(m.w, o.w)));
+  };
+  auto v_field4 = [&](int key) {
+    const uint4 m = *reinterpret_cast<const uint4 *>(&vmx[key]);
+    return make_uint4(exp_field(m.x), exp_field(m.y), exp_field(m.z), exp_field(m.w));
+  };
+  auto write_tile = [&]() {
+    if (tid < KT / 4) {
+      const uint4 k = k_field4(4 * tid), v = v_field4(4 * tid);
+      *reinterpret_cast<int4 *>(&kex[4 * tid]) = make_int4(plane_exp(k.x), plane_exp(k.y), plane_exp(k.z), plane_exp(k.w));
+      *reinterpret_cast<uint4 *>(&vpw[4 * tid]) = v;
+    }
+    uint4 *dst;
+    int plane;
+    float sk[4], sv[8];  // plane scales of the keys
+    if (isk) {
+      dst = kf + ((kkey >> 5) * T::DS + (kdim >> 4)) * 64 + (kkey & 31) + 4 * (kdim & 8);
+      plane = T::KF;
+      const uint4 f = k_field4(kkey);
+      sk[0] = plane_scale(f.x), sk[1] = plane_scale(f.y), sk[2] = plane_scale(f.z), sk[3] = plane_scale(f.w);
+    } else {
+      dst = vf + ((vch >> 5) * T::KS + (vkey >> 4)) * 64 + (vch & 31) + 8 * (vkey & 4);
+      plane = T::VF;
 #pragma unroll
-    for (int j = 0; j < T::NU; ++j) {
-      const int u = unit_of(j);
-      if (u >= 2 * T::UK) continue;
-      const bool isk = u - lane < T::UK;
-      const int x = isk ? u : u - T::UK;
-      uint4 *dst;
-      int plane;
-      if (isk) {
-        const int key = 4 * (x % (KT / 4)), o = x / (KT / 4);
-        dst = kf + ((key >> 5) * T::DS + (o >> 1)) * 64 + (key & 31) + 32 * (o & 1);
-        plane = T::KF;
-      } else {
-        const int ch = 4 * (x % (DP / 4)), kk = x / (DP / 4);
-        dst = vf + ((ch >> 5) * T::KS + (kk >> 1)) * 64 + (ch & 31) + 32 * (kk & 1);
-        plane = T::VF;
+      for (int e = 0; e < 8; e += 4) {
+        const uint4 f = v_field4(vkey + 2 * e);
+        sv[e] = plane_scale(f.x), sv[e + 1] = plane_scale(f.y), sv[e + 2] = plane_scale(f.z), sv[e + 3] = plane_scale(f.w);
       }
-      const float s = isk ? ks : vs;
+    }
+    if (spare) return;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v[8];
+    for (int i = 0; i < 4; ++i) {
+      float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          v[e] = i == 0 ? raw[j][e].x : (i == 1 ? raw[j][e].y : (i == 2 ? raw[j][e].z : raw[j][e].w));
-        planes8(v, s, dst[i], dst[plane + i]);
-      }
+      for (int e = 0; e < 8; ++e) v[e] = i == 0 ? raw[e].x : (i == 1 ? raw[e].y : (i == 2 ? raw[e].z : raw[e].w));
+      if (isk) planes8(v, sk[i], dst[i], dst[plane + i]);
+      else planes8(v, sv, dst[i], dst[plane + i]);
     }
   };
 
@@ -342,36 +413,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     for (int e = 0; e < 16; ++e) acc[c][e] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;  // l_run: this half-wave's keys
   bool slow = false;
-  int ev = -110;                          // exponent of V's planes, acc holds O 2^(kPExp - ev)
+  // A row's weights of a tile's values are w = p 2^(the key's V exponent), in
+  // planes of the row's own scale: by the largest w up to this tile, falling as
+  // the running maximum of the scores leaves them behind.
+  float w_run = 0.0f;  // acc holds O 2^28 / (its power of two, at least 2^-112)
 
   if (tb < te) load_tile(tb);
   for (int t = tb; t < te; ++t) {
-    const int par = t & 1;
     trim_tile(t);
+    key_maxima();
+    __syncthreads();  // the maxima, and every wave is done with the previous tile's fragments
     {
-      uint32_t mk, mv;
-      wave_max(mk, mv);
-      if (lane == 0) {
-        red[par][0][wave] = qbad ? kInfBits : mk;
-        red[par][1][wave] = mv;
+      const uint4 f = *reinterpret_cast<const uint4 *>(bad);
+      if (f.x | f.y | f.z | f.w) {  // uniform: an infinity or NaN among the keys or in q
+        slow = true;
+        break;
       }
     }
-    __syncthreads();  // the maxima, and every wave is done with the previous tile's fragments
-    uint32_t mk = max(max(red[par][0][0], red[par][0][1]), max(red[par][0][2], red[par][0][3]));
-    uint32_t mv = max(max(red[par][1][0], red[par][1][1]), max(red[par][1][2], red[par][1][3]));
-    if (mk >= kInfBits || mv >= kInfBits) {  // uniform: an infinity or NaN among the keys or in q
-      slow = true;
-      break;
-    }
-    const int ek = plane_exp(mk), ev_new = max(ev, plane_exp(mv));
-    write_tile(ldexpf(1.0f, -ek), ldexpf(1.0f, -ev_new));
+    write_tile();
     if (t + 1 < te) load_tile(t + 1);
     __syncthreads();
 
     float s[T::KB][16];
     if (busy) {
       // ---- scores of this lane's row: keys 32 kb + 8 (i / 4) + 4 h + i % 4
-      const float cf = ldexpf(qscale, ek);
       // (Fragments are read one step ahead of their products.)
       uint4 fh[2], fl[2];
       fh[0] = kf[lane];
@@ -390,7 +455,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         d = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh8, qh[ds], d, 0, 0, 0);
         if (ds == T::DS - 1) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s[kb][i] = d[i] * cf;
+          for (int i = 0; i < 16; i += 4) {
+            const int4 ke = *reinterpret_cast<const int4 *>(&kex[32 * kb + 2 * i + 4 * h]);
+            s[kb][i] = ldexpf(d[i], qexp + ke.x);
+            s[kb][i + 1] = ldexpf(d[i + 1], qexp + ke.y);
+            s[kb][i + 2] = ldexpf(d[i + 2], qexp + ke.z);
+            s[kb][i + 3] = ldexpf(d[i + 3], qexp + ke.w);
+          }
           d = f32x16{};
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -426,18 +497,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       const float m_new = fmaxf(m_run, mx);
       const float m_sub = m_new == -INFINITY ? 0.0f : m_new;  // no key yet: every p is exp(-inf) = 0
       const float keep = __expf(m_run - m_sub);
-      float sum = 0.0f;
+      float sum = 0.0f, wmx = 0.0f;
 #pragma unroll
       for (int kb = 0; kb < T::KB; ++kb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          s[kb][i] = __expf(s[kb][i] - m_sub);
-          sum += s[kb][i];
+        for (int i = 0; i < 16; i += 4) {
+          const float4 vs = *reinterpret_cast<const float4 *>(&vpw[32 * kb + 2 * i + 4 * h]);
+          const float ve[4] = {vs.x, vs.y, vs.z, vs.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float p = __expf(s[kb][i + e] - m_sub);
+            sum += p;
+            s[kb][i + e] = p * ve[e];
+            wmx = fmaxf(wmx, s[kb][i + e]);
+          }
         }
       l_run = l_run * keep + sum;
       m_run = m_new;
-      // acc to the new maximum and V's new exponent (skipped when no row changes)
-      const float f = ldexpf(keep, max(ev - ev_new, -200));
+      wmx = fmaxf(wmx, dev::xor_lanes<32>(wmx));
+      const uint32_t w_old = exp_field(__float_as_uint(w_run));
+      w_run = fmaxf(w_run * keep, wmx);
+      const uint32_t w_new = exp_field(__float_as_uint(w_run));
+      const float wscale = plane_scale(w_new);
+      // acc to the new maximum and the new scale (skipped when no row changes)
+      const float f = ldexpf(keep, (int(w_old) - int(w_new)) >> 23);
       if (__ballot(f != 1.0f) != 0) {
 #pragma unroll
         for (int c = 0; c < T::CB; ++c)
@@ -451,7 +534,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
         for (int e = 0; e < 8; ++e) pv[e] = s[ks >> 1][8 * (ks & 1) + e];
         uint4 ph, pl;
-        planes8(pv, 16384.0f, ph, pl);
+        planes8(pv, wscale, ph, pl);
         p_h[ks & 1] = as_half8(ph);
         p_l[ks & 1] = as_half8(pl);
       };
@@ -475,7 +558,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    ev = ev_new;
   }
   if (slow) {
     // Infinities or NaNs among the keys would reach rows that do not see them
@@ -523,6 +605,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
   if (!qin || !busy) return;
   const float l = l_run + dev::xor_lanes<32>(l_run);
+  const int oexp = int(exp_field(__float_as_uint(w_run)) >> 23) - (127 + 28);
   const size_t row_head = size_t(r) * a.heads + head;
   const bool whole = a.splits == 1;
   float *o = whole ? a.out + row_head * a.dim : a.opart + (size_t(split) * a.rows * a.heads + row_head) * a.dim;
@@ -535,7 +618,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] = ldexpf(acc[c][4 * g + e], ev - kPExp);
+        v[e] = ldexpf(acc[c][4 * g + e], oexp);
         if (whole) v[e] = v[e] / l;
       }
       if (cvec) {
@@ -582,9 +665,8 @@ bool attn_mm_plan(AttnPlan &p, int rows, int cap, int heads, int kv_heads, int d
   // The keys of one workgroup's rows: at most the window and those rows.
   const int longest = window > 0 ? int(std::min<long long>((long long)window + kQRows, last_end)) : last_end;
   const int tiles = (longest + 63) / 64;
-  // Two workgroups per CU (one where a tile is 64 keys of 96 channels, which
-  // takes a SIMD's registers), at least two tiles of 64 keys each.
-  const long long wgs = (long long)kv_heads * p.qtiles, target = std::max(1, tuning().attn_wgs) / (dim > 64 && dim <= 96 ? 2 : 1);
+  // Two workgroups per CU, at least two tiles of 64 keys (four of 32) each.
+  const long long wgs = (long long)kv_heads * p.qtiles, target = std::max(1, tuning().attn_wgs);
   p.splits = int(std::max<long long>(1, std::min<long long>(target / std::max<long long>(1, wgs), tiles / 2)));
   p.part_floats = p.splits > 1 ? size_t(p.splits) * rows * heads * (size_t(dim) + 2) : 0;
   return true;
@@ -613,7 +695,7 @@ void attn_mm_launch(const float *q, const float *cache, float *out, float *opart
   a.softcap = softcap;
   a.scale = scale;
   if (dim <= 64) launch<64, 64>(a, s);
-  else if (dim <= 96) launch<96, 64>(a, s);
+  else if (dim <= 96) launch<96, 32>(a, s);
   else launch<128, 32>(a, s);
   hip_check(hipGetLastError(), "attention launch");
 }

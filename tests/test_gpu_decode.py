@@ -370,6 +370,42 @@ def test_attention_of_many_rows(ctx, rng, tune, case):
         ctx.Recycle(z)
 
 
+@pytest.mark.parametrize("dim", [64, 80, 128])
+@pytest.mark.parametrize("where", ["mask", "some rows", "later", "window"])
+@pytest.mark.parametrize("size", [1e6, 1e8, 1e12, 1e30])
+def test_attention_of_many_rows_hidden_keys(ctx, rng, tune, dim, where, size):
+    """A key that a row does not see may hold anything finite: by the mask (for all rows, or some), by a later
+    position, behind the window.  Every key's K and V have planes of their own scale, so the row's result keeps the
+    bounds of test_attention_of_many_rows.  Rows that do see such a key give it all the weight or none (its score is
+    1e5 and more away from the others), so they keep them, too."""
+    rows, heads, kvh, cap, pos = 48, 8, 2, 200, 100
+    window = 60 if where == "window" else 0
+    masked = where in ("mask", "some rows")
+    q, cache = many_inputs(rng, (rows, heads, kvh, dim, cap, pos, window, 0.0, 0.0, masked))
+    hidden = {"mask": (3, 70), "some rows": (31, 64), "later": (pos + 20,), "window": (pos - 30,)}[where]
+    kt, vs = cache[:kvh * dim * cap].reshape(kvh, dim, cap), cache[kvh * dim * cap:2 * kvh * dim * cap].reshape(kvh, cap, dim)
+    for key in hidden:
+        kt[:, :, key] = rng.standard_normal((kvh, dim)) * size
+        vs[:, key] = rng.standard_normal((kvh, dim)) * size
+    if masked:
+        m = cache.view(np.uint32)[2 * cap * kvh * dim:].reshape(rows, cap)
+        m[:, hidden] = 0
+        if where == "some rows":
+            m[::2, hidden[0]] = m[::3, hidden[1]] = 1
+    want = oracle.cached_attention(q, cache, rows, cap, heads, kvh, dim, pos, window, 0.0, 0.0, masked)
+    want = want.reshape(rows * heads, dim)
+    tq, tc, to = up(ctx, q), up(ctx, cache), ctx.NewTensor(rows * heads * dim)
+    for mm, wgs in (("0", "512"), ("1", "512"), ("1", "1")):
+        tune("QNN_ATTN_MM", mm)
+        tune("QNN_ATTN_WGS", wgs)
+        ctx.CachedAttention(to, tq, tc, rows, cap, heads, kvh, dim, pos, window, 0.0, 0.0, masked)
+        got = ctx.Download(to).reshape(rows * heads, dim)
+        for i in range(rows * heads):
+            assert normwise_rel_err(got[i], want[i]) <= 1e-5, (mm, wgs, i)
+    for z in (tq, tc, to):
+        ctx.Recycle(z)
+
+
 @pytest.mark.parametrize("where", ["k", "v"])
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
 def test_attention_of_many_rows_infinite_keys(ctx, rng, tune, where, value):
