@@ -45,8 +45,8 @@
 // rows over 4096 keys 453 -> 63 us, over 16384 keys 1900 -> 160, 64 rows 224 ->
 // 48, 16 rows 72 -> 31, 8 rows 45 -> 30 us (scales per tile and not per key: 1 to
 // 3 us less, all in the two larger).  One against two workgroups per CU: 69
-// against 65 us, 192 against 160; with four, 77 and 170.  Error against 64 bits
-// 5.9e-7 -> 3.4e-7; over 60 drawn shapes that come here 0.74 to 0.84 of k_attn's.
+// against 65 us, 192 against 160 (four: 170).  Error against 64 bits 5.9e-7 ->
+// 3.4e-7; over 60 drawn shapes that come here 0.74 to 0.84 of k_attn's.
 // From when (attn_mm_plan): four rows, and rows x heads x keys of 512 k: 4
 // rows of 32 heads over 4096 keys 31.2 -> 29.1 us, 2 rows 27.1 -> 30.6 (over
 // 16384 keys 49.3 -> 63.2); 32 rows of 16 heads over 512 keys 26.0 -> 29.9,
@@ -665,9 +665,13 @@ bool attn_mm_plan(AttnPlan &p, int rows, int cap, int heads, int kv_heads, int d
   // The keys of one workgroup's rows: at most the window and those rows.
   const int longest = window > 0 ? int(std::min<long long>((long long)window + kQRows, last_end)) : last_end;
   const int tiles = (longest + 63) / 64;
-  // Two workgroups per CU, at least two tiles of 64 keys (four of 32) each.
+  // Two workgroups per CU, at least two tiles of 64 keys (four of 32) each, and
+  // four while there is a workgroup for every CU (shorter parts cost the merge
+  // more than they save: 128 rows of 16 heads on 8, dim 96, over 3000 keys in 16
+  // parts 42, in 23 45 us; 64 rows of 32 on 8, dim 128, over 4096 in 16 45.5, in 32 47.5).
   const long long wgs = (long long)kv_heads * p.qtiles, target = std::max(1, tuning().attn_wgs);
-  p.splits = int(std::max<long long>(1, std::min<long long>(target / std::max<long long>(1, wgs), tiles / 2)));
+  const long long longer = std::max<long long>(tiles / 4, target / 2 / wgs);
+  p.splits = int(std::max<long long>(1, std::min<long long>({target / wgs, tiles / 2, longer})));
   p.part_floats = p.splits > 1 ? size_t(p.splits) * rows * heads * (size_t(dim) + 2) : 0;
   return true;
 }
