@@ -689,7 +689,10 @@ void run_int4(qnn_ctx_s *ctx, const WeightEntry *w, const WeightEntry *w2, int m
               int rows, int in_dim, int out_dim, const float *prob, float *g_out = nullptr, float *u_out = nullptr,
               const FixedWs *fixed = nullptr) {
   const I4Layout &l = w->i4;
-  if (mode != I4_ACCUM && int4_gemm_applies(l, rows)) {
+  // (A gate/up launch of the GEMM writes both sums: the one-row SwiGLU, which
+  // has no tensors for them, stays with the matvec that its workspace was sized
+  // for, whatever QNN_I4_GEMM_ROWS says.)
+  if ((mode == I4_STORE || (mode == I4_SWIGLU && g_out && u_out)) && int4_gemm_applies(l, rows)) {
     I4Launch a;
     a.l = l;
     a.nib = w->dptr;

@@ -476,6 +476,7 @@ bool int4_gemm_applies(const I4Layout &l, int rows) {
 
 void int4_gemm_launch(const I4Launch &a, const I4GemmPlan &p, uint8_t *ws, hipStream_t s) {
   const bool pair = a.mode == I4_SWIGLU;
+  if (pair && (!a.g_out || !a.u_out || !a.nib2)) fail(QNN_E_INVALID_OP, "int4 gemm pair without both matrices and sums");
   I4GemmArgs g;
   g.l = a.l;
   g.w[0] = static_cast<const uint8_t *>(a.nib);

@@ -251,3 +251,27 @@ def test_many_rows_pair_equals_separate(ctx, rng, tune, rows, hidden, inter, int
     for a, b in zip(got["1"], got["0"]):
         assert np.array_equal(a, b)
     ctx.Recycle(x)
+
+
+@pytest.mark.parametrize("down", [True, False])
+def test_one_row_swiglu_with_the_gemm_from_one_row(ctx, rng, tune, down):
+    """QNN_I4_GEMM_ROWS=1 sends one-row Int4Linear calls to the GEMM.  A gate/up SwiGLU has no tensors for the two sums
+    that the GEMM writes, so launched on its own (the next call is not its down projection) or fused, it is what it is
+    with the default, to the bit."""
+    from quicknn_amd import hip
+
+    hidden, inter = 512, 1536
+    g, u = hip.MemoryBlock.int4(rand_int4(rng, inter, hidden)), hip.MemoryBlock.int4(rand_int4(rng, inter, hidden))
+    d = hip.MemoryBlock.int4(rand_int4(rng, hidden, inter))
+    x = ctx.UploadRaw(rng.standard_normal(hidden).astype(np.float32))
+    h, y = ctx.NewTensor(inter), ctx.NewTensor(hidden)
+    got = {}
+    for rows in ("25", "1"):
+        tune("QNN_I4_GEMM_ROWS", rows)
+        assert ctx.TrySwiGLUVector(h, x, g, u, hidden, inter)
+        if down:
+            ctx.Int4Linear(y, h, d, 1, inter, hidden)
+        got[rows] = ctx.Download(h).view(np.uint32).copy()
+    assert np.array_equal(got["25"], got["1"])
+    for t in (x, h, y):
+        ctx.Recycle(t)
