@@ -514,16 +514,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TT == 1 ? 4
   const int bw_ = DOWN ? item * 4 + (wave >> 1) : item, b = min(bw_, l.blocks - 1);  // past the last: not written
   const int ch0 = kq * chunks / KQ, ch1 = (kq + 1) * chunks / KQ;
   const uint8_t *wb = DOWN ? a.down + size_t(e) * a.dn_stride : a.gate_up + size_t(2 * e + mat) * a.gu_stride;
-  // One block's weights: steps past the last read zeros (scale pieces hold zeros there).
+  // One block's weights.  Steps past the last read zeros (scale pieces hold
+  // zeros there): the whole offset is the lane's, as a scalar offset need not
+  // take part in the range check, and the last expert's down matrix has less
+  // behind its nibbles than such a step could reach.
   const dev::Rsrc nr = dev::rsrc(wb + size_t(b) * l.steps * 1024, size_t(l.steps) * 1024);
   const dev::Rsrc sr = dev::rsrc(wb + l.nib_bytes() + size_t(b) * l.quads() * 1024, size_t(l.quads()) * 1024);
   const dev::Rsrc xr = DOWN ? dev::rsrc(mm.hfrag, size_t(a.rows) * a.topk * gpad * 128)
                             : dev::rsrc(mm.xfrag, size_t(a.rows) * gpad * 128);
   const int p = lane & 15, d = lane >> 4;
   auto load_w = [&](MmWeights &m, int ch) {
+    const uint32_t at = uint32_t(lane) * 16u + uint32_t(ch) * 4096u;
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      m.w[g] = dev::ld128<dev::kStream>(nr, uint32_t(lane) * 16u, uint32_t(ch * 4 + g) * 1024u);
+    for (int g = 0; g < 4; ++g) m.w[g] = dev::ld128<dev::kStream>(nr, at + uint32_t(g) * 1024u, 0u);
     m.q = dev::ld128<dev::kStream>(sr, uint32_t(lane) * 16u, uint32_t(ch) * 1024u);
   };
   const dev::I4Masks masks = dev::i4_masks();
