@@ -46,6 +46,7 @@ struct qnn_ctx_s {
   qnn_tensor_s *scratch[4] = {nullptr, nullptr, nullptr, nullptr};
   std::unordered_map<std::string, qnn::WeightEntry *> weights;
   uint64_t weight_bytes = 0, weight_limit = 0, clock = 0;
+  bool few_row_copies = true;  // false once device memory had no room for an optional fp16 copy
   int *error_flag = nullptr;
   // split-K workspace: partial sums + per-tile tickets (zeroed once, self-resetting)
   float *partial = nullptr;
@@ -367,11 +368,14 @@ std::string weight_key(const char *kind, const qnn_weight *w, uint64_t bytes) {
   return buf;
 }
 
-void evict_one_or_fail(qnn_ctx_s *ctx) {  // EvictOne (QuickNN.Vulkan.pas:551-579): LRU of unpinned entries
+// EvictOne (QuickNN.Vulkan.pas:551-579): LRU of unpinned entries, copies made
+// on the device before weights, which come back from the host only.
+void evict_one_or_fail(qnn_ctx_s *ctx) {
   qnn::WeightEntry *oldest = nullptr;
   for (auto &kv : ctx->weights) {
     auto *e = kv.second;
-    if (e->pins == 0 && e->op_pins == 0 && (!oldest || e->last_use < oldest->last_use)) oldest = e;
+    if (e->pins != 0 || e->op_pins != 0) continue;
+    if (!oldest || (e->derived != oldest->derived ? e->derived : e->last_use < oldest->last_use)) oldest = e;
   }
   if (!oldest) fail(QNN_E_RANGE, "VRAM cache cannot hold the active chain");
   if (ctx->on_evicted && !oldest->derived) ctx->on_evicted(oldest->identity, ctx->on_evicted_user);
@@ -985,12 +989,14 @@ bool try_fused_mlp(qnn_ctx_s *ctx, WeightEntry *d, float *y) {
 int q8_gemm_min_rows() { return std::max(2, tuning().q8_gemm_min_rows); }
 
 // The fp16 copy of a resident GGUF weight for the GEMM (k_h16_gemm), found or
-// made on the device: a cache entry of its own (key + "/h16"), evicted like
-// any other (its eviction is not reported).  A Q8_0 copy scales by the
+// made on the device: a cache entry of its own (key + "/h16"), evicted before
+// any weight (its eviction is not reported).  A Q8_0 copy scales by the
 // weight's own row exponents; a copy of any other encoding carries its row
 // exponents after the values.  Null under graph capture when it does not
-// exist yet (making it allocates).
-WeightEntry *h16_entry(qnn_ctx_s *ctx, const WeightEntry *w) {
+// exist yet (making it allocates), and where a copy that is not `needed` finds
+// no device memory (it evicts nothing for want of it; further ones are then
+// not tried).
+WeightEntry *h16_entry(qnn_ctx_s *ctx, const WeightEntry *w, bool needed) {
   const std::string key = w->key + "/h16";
   if (WeightEntry *h = lookup(ctx, key)) return h;
   if (ctx->capturing) return nullptr;
@@ -1004,7 +1010,14 @@ WeightEntry *h16_entry(qnn_ctx_s *ctx, const WeightEntry *w) {
   e->bytes = vbytes + (own_exp ? (size_t(w->gg.rows) * 4 + 255) / 256 * 256 : 0);
   e->source_bytes = 0;
   try {
-    e->dptr = alloc_weight(ctx, e->bytes);
+    if (needed) {
+      e->dptr = alloc_weight(ctx, e->bytes);
+    } else if (hipMalloc(&e->dptr, e->bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->few_row_copies = false;
+      delete e;
+      return nullptr;
+    }
     if (own_exp) {
       int *ew = reinterpret_cast<int *>(static_cast<uint8_t *>(e->dptr) + vbytes);
       gguf_rowexp_launch(w->gg, w->dptr, ew, w->gg.rows, ctx->stream);
@@ -1030,7 +1043,8 @@ int gemm_max_rows(int in_dim) {
 }
 
 // Fewer rows than QNN_GEMM_H16 (from q8_gemm_min_rows on) take the fp16 copy
-// too where it is there or costs no other weight its place: 8 rows of 3072 ->
+// too where it is there or costs no other weight its place, when it is made
+// (it fits beside what is resident) and later (it goes before any weight): 8 rows of 3072 ->
 // 12288 take 18.0 us over the copy, 36.5 decoding; of 4096 -> 4096 19.5 and
 // 49.7; 64 rows 19.1 and 39.1, 20.4 and 52.0.  Weights below 1 M elements keep
 // decoding: their copy takes longer to make (30 us and more) than a few such
@@ -1039,7 +1053,8 @@ bool few_rows_take_copy(qnn_ctx_s *ctx, const WeightEntry *w, int rows, size_t c
   if (w->gg.enc != QNN_WE_Q8_0 || tuning().gemm_h16 <= 0 || rows < q8_gemm_min_rows() ||
       int64_t(w->gg.rows) * w->gg.cols < (1 << 20))
     return false;
-  return ctx->weight_bytes + copy_bytes <= ctx->weight_limit || ctx->weights.count(w->key + "/h16") != 0;
+  return (ctx->few_row_copies && ctx->weight_bytes + copy_bytes <= ctx->weight_limit) ||
+         ctx->weights.count(w->key + "/h16") != 0;
 }
 
 // Multi-row GGUF projection.  From QNN_GEMM_H16 rows (Q8_0; fewer:
@@ -1062,7 +1077,7 @@ bool run_gguf_gemm(qnn_ctx_s *ctx, WeightEntry *w, const float *x, float *y, int
     w->op_pins++;  // making the copy may evict: not the weight it is made from
     WeightEntry *h = nullptr;
     try {
-      h = h16_entry(ctx, w);
+      h = h16_entry(ctx, w, rows >= from);
     } catch (...) {
       w->op_pins--;
       throw;

@@ -209,3 +209,33 @@ def test_few_rows_make_no_fp16_copy_by_eviction(small, tune):
     assert ctx.status().weight_evictions > s1.weight_evictions and ctx.status().gemm_h16 == s1.gemm_h16 + 1
     for t in (a, y, x, y1):
         ctx.Recycle(t)
+
+
+def test_uploads_evict_fp16_copies_before_weights(small, tune):
+    """A copy can be made again on the device, a weight has to come from the host: where room is needed the copies go
+    first, however recently used, and the weights that they were made from stay (in a cache that holds the weights
+    of a model but not their copies, a pass that uploads them one by one makes copies of the first ones)."""
+    from quicknn_amd import hip
+
+    ctx = small
+    m, k, n = 8, 1024, 2048
+    rng = np.random.default_rng(10)
+    ws = [hip.MemoryBlock.gguf(hip.gguf_quantize(hip.WE_Q8_0, (rng.standard_normal(n * k) * 0.02).astype(np.float32)),
+                               n, k, hip.WE_Q8_0) for _ in range(2)]
+    a, y = ctx.UploadRaw(rng.standard_normal((m, k)).astype(np.float32)), ctx.NewTensor(m * n)
+    x1, y1 = ctx.UploadRaw(rng.standard_normal(k).astype(np.float32)), ctx.NewTensor(n)
+    tune("QNN_GEMM_H16", "4")  # a copy whatever it evicts: earlier tests left the cache full
+    ctx.Linear(y, a, ws[0], None, None, m, k, n)
+    first = ctx.Download(y).copy()
+    tune("QNN_GEMM_H16", "128")
+    seen = []
+    ctx.OnWeightEvicted = seen.append
+    ctx.Linear(y1, x1, ws[1], None, None, 1, k, n)  # 2.2 MB more than there is room for
+    ctx.Download(y1)
+    ctx.OnWeightEvicted = None
+    assert seen == [] and ctx.IsWeightResident(ws[0], n, k) and ctx.IsWeightResident(ws[1], n, k)
+    h = ctx.status().gemm_h16
+    ctx.Linear(y, a, ws[0], None, None, m, k, n)  # no copy any more, and no room for one: the same bits
+    assert np.array_equal(ctx.Download(y).view(np.uint32), first.view(np.uint32)) and ctx.status().gemm_h16 == h
+    for t in (a, y, x1, y1):
+        ctx.Recycle(t)
