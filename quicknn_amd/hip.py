@@ -245,15 +245,6 @@ def float_bits(v: float) -> int:
 _identity = itertools.count(1)
 
 
-def _address(a: np.ndarray) -> int:
-    """``a.ctypes.data``, which builds an interface object on each use (2.2 us, a third of an op's host time); through
-    the buffer protocol 0.6.  What that refuses (read-only, empty, strided arrays) takes the property."""
-    try:
-        return ctypes.addressof(ctypes.c_char.from_buffer(a))
-    except (TypeError, ValueError, BufferError):
-        return a.ctypes.data
-
-
 _int_arrays: dict = {}  # length -> ctypes array type
 
 
@@ -276,7 +267,7 @@ class MemoryBlock:
 
     def __init__(self, data: np.ndarray, shape, dtype: int, encoding: int = WE_NATIVE, offset: int = 0,
                  size: int | None = None, identity: int | None = None):
-        self.data = np.ascontiguousarray(data)
+        self.data = data
         self.shape = tuple(int(s) for s in shape)
         self.dtype = dtype
         self.encoding = encoding
@@ -284,8 +275,19 @@ class MemoryBlock:
         self.size = int(size if size is not None else int(np.prod(self.shape)))
         self.identity = identity if identity is not None else next(_identity)
 
+    @property
+    def data(self) -> np.ndarray:
+        return self._data
+
+    @data.setter
+    def data(self, values: np.ndarray) -> None:
+        # The address is taken here, once: `ctypes.data` builds an interface object on each use (1.1 us on the host of
+        # every weight operation, read-only arrays and mappings included).
+        self._data = np.ascontiguousarray(values)
+        self._address = self._data.ctypes.data
+
     def desc(self) -> _Weight:
-        return _Weight(self.identity, _address(self.data), self.offset, self.size, self.shape[0],
+        return _Weight(self.identity, self._address, self.offset, self.size, self.shape[0],
                        self.shape[1] if len(self.shape) > 1 else 1, self.dtype, self.encoding)
 
     @staticmethod

@@ -94,3 +94,38 @@ def test_pascal_unit_binds_every_entry_point():
     assert not missing, missing
     wrong = {n: (pas[n], c[n]) for n in c if pas[n] != c[n]}
     assert not wrong, wrong
+
+
+@pytest.mark.parametrize("kind", ["owned", "read-only", "mapped", "empty", "transposed"])
+def test_weight_descriptor_address(tmp_path, kind):
+    """A descriptor holds the address of the block's own (contiguous) storage, also after `data` is replaced, and
+    building one raises and catches nothing: it is done for every weight operation, on mappings as on arrays."""
+    import sys
+
+    import numpy as np
+
+    from quicknn_amd import hip
+
+    a = np.arange(24, dtype=np.uint8).reshape(4, 6)
+    if kind == "read-only":
+        a.setflags(write=False)
+    elif kind == "mapped":
+        (tmp_path / "w").write_bytes(a.tobytes())
+        a = np.memmap(tmp_path / "w", np.uint8, "r", shape=(4, 6))
+    elif kind == "empty":
+        a = a[:0]
+    elif kind == "transposed":
+        a = a.T
+    block = hip.MemoryBlock(a, a.shape, hip.DT_U8)
+    events = []
+    sys.setprofile(lambda frame, event, arg: events.append(event))
+    try:
+        desc = block.desc()
+    finally:
+        sys.setprofile(None)
+    assert desc.data == block.data.ctypes.data and block.data.flags.c_contiguous
+    assert "c_exception" not in events and "exception" not in events
+    if kind not in ("empty", "transposed"):
+        assert desc.data == a.ctypes.data
+    block.data = np.ones(24, np.uint8)
+    assert block.desc().data == block.data.ctypes.data
