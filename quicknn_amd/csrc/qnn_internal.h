@@ -327,7 +327,7 @@ struct MoEGemm {
   int gpad_x = 0, gpad_h = 0;
 };
 struct MoEPlanSizes {
-  int slots = 0, mt = 1, gsw = 4, slices_gu = 1, slices_dn = 1, sps_gu = 1, sps_dn = 1;
+  int slots = 0, gsw = 4, slices_gu = 1, slices_dn = 1, sps_gu = 1, sps_dn = 1;
   size_t lds_gu = 0, lds_dn = 0;  // dynamic LDS per launch
   size_t partial_floats = 0, counters = 0;
   size_t plan_words = 0;  // slot plans of the multi-token launches (k_moe_plan)

@@ -246,10 +246,10 @@ __device__ void load_plan(MoEPlan &pl, const MoELaunch &a, int n, int slot, int 
 // launch (a tile is one block) + expert combine.  A workgroup is one tile of
 // one slot and a K-slice of 4*sps steps; wave w takes steps [w*sps, (w+1)*sps)
 // of it and the four partial sums meet in LDS in wave order.
-template <int MT, int GSW, bool DOWN>
+template <int GSW, bool DOWN>
 __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices, const int sps, const int slots) {
   extern __shared__ uint4 dyn_lds[];
-  __shared__ float red[3][MT][64];
+  __shared__ float red[3][64];
   // Expert layouts have one lane per row (int4_layout(.., true)), so a
   // slice is at most 4 x 8 x 32 elements: one pass of activation loads
   // (x_iters<2>), 12 fewer VGPRs than the lanes-per-row general form.
@@ -299,10 +299,10 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
     const int R = pl.pos[min(m, c - 1)];
     return DOWN ? uint32_t(R) * uint32_t(a.inter) * 4u : uint32_t(R / a.topk) * uint32_t(a.hidden) * 4u;
   };
-  float4 xr[MT][dev::x_iters<XG>()];
-  dev::load_x<MT, XG>(xr, xsrc, xoff, min(c, MT), ws0 * L * 32, sgroups * 32, tid);
-  const dev::XPlanes xs = dev::xplanes_at(dyn_lds, MT, 4 * sps * L);
-  // The first chunk's activations are requested, then the weights, then the
+  float4 xr[1][dev::x_iters<XG>()];  // one position's activations
+  dev::load_x<1, XG>(xr, xsrc, xoff, 1, ws0 * L * 32, sgroups * 32, tid);
+  const dev::XPlanes xs = dev::xplanes_at(dyn_lds, 1, 4 * sps * L);
+  // The first position's activations are requested, then the weights, then the
   // activations are staged (waiting for them alone).  With the plan loaded
   // rather than built this order is the fastest (batch 16: 92.5 -> 89.6 us
   // against staging before the weight loads are issued; weights first:
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
     dev::load_w<GSW>(w, sc, dev::rsrc(wbase, wbytes), dev::rsrc(wbase + l.nib_bytes(), wbytes - l.nib_bytes()), l, b,
                      s0, wl, moff, moff);
   __builtin_amdgcn_sched_barrier(0);  // every load issued before the staging waits for x
-  dev::stage_x<MT, XG>(xs, xr, min(c, MT), ws0 * L * 32, sgroups * 32, kin, tid, lane);
+  dev::stage_x<1, XG>(xs, xr, 1, ws0 * L * 32, sgroups * 32, kin, tid, lane);
 
   dev::XPlanes xw = xs;  // this wave's groups
   xw.q = xs.q + size_t(wave) * sps * L * dev::kXWords;
@@ -338,21 +338,18 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
     }
   };
 
-  for (int m0 = 0; m0 < c; m0 += MT) {
-    if (m0 > 0) {
-      __syncthreads();  // the previous chunk's LDS reads are done
-      dev::stage_x<MT, XG>(xs, xr, min(c - m0, MT), ws0 * L * 32, sgroups * 32, kin, tid, lane);
+  for (int m = 0; m < c; ++m) {
+    if (m > 0) {
+      __syncthreads();  // the previous position's LDS reads are done
+      dev::stage_x<1, XG>(xs, xr, 1, ws0 * L * 32, sgroups * 32, kin, tid, lane);
     }
     __syncthreads();
-    // The next chunk's activations are requested now (its staging is done
-    // with these registers), so their latency overlaps this chunk's products
+    // The next position's activations are requested now (its staging is done
+    // with these registers), so their latency overlaps this one's products
     // and part sums instead of following them (batch 16: 101.5 -> 100.9 us).
-    if (m0 + MT < c)
-      dev::load_x<MT, XG>(xr, xsrc, [&](int m) { return xoff(m0 + MT + m); }, min(c - m0 - MT, MT), ws0 * L * 32,
-                           sgroups * 32, tid);
-    float acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = 0.0f;
+    if (m + 1 < c)
+      dev::load_x<1, XG>(xr, xsrc, [&](int) { return xoff(m + 1); }, 1, ws0 * L * 32, sgroups * 32, tid);
+    float acc[1] = {0.0f};
     if (ns > 0) {
       // The weights are unpacked inside every token pass: hoisted out of the
       // pass loop (the compiler's choice) the unpacked nibbles of all steps
@@ -361,24 +358,16 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
       // token, so one pass).
 #pragma unroll
       for (int g = 0; g < GSW; ++g) asm volatile("" : "+v"(w[g].x), "+v"(w[g].y), "+v"(w[g].z), "+v"(w[g].w));
-      dev::dot<MT, GSW>(acc, w, sc, xw, L, j, ns);
-      dev::reduce_lanes<MT>(acc, L);
+      dev::dot<1, GSW>(acc, w, sc, xw, L, j, ns);
+      dev::reduce_lanes<1>(acc, L);
     }
-    if (wave > 0) {
-#pragma unroll
-      for (int m = 0; m < MT; ++m) red[wave - 1][m][lane] = acc[m];
-    }
+    if (wave > 0) red[wave - 1][lane] = acc[0];
     __syncthreads();
     if (wave == 0) {
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        acc[m] = ((acc[m] + red[0][m][lane]) + red[1][m][lane]) + red[2][m][lane];
-        if (m0 + m < c) {
-          const int R = pl.pos[m0 + m];
-          if (slices > 1) dev::xstore(part + size_t(R) * 64, acc[m]);
-          else finish(R, acc[m]);
-        }
-      }
+      const float v = ((acc[0] + red[0][lane]) + red[1][lane]) + red[2][lane];
+      const int R = pl.pos[m];
+      if (slices > 1) dev::xstore(part + size_t(R) * 64, v);
+      else finish(R, v);
     }
   }
   if (!DOWN && wave > 0) return;
@@ -394,13 +383,10 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
       last = dev::last_arrival(ctr, unsigned(slices), lane);
       if (last) {
         const float *pt = a.partial + size_t(tile) * slices * n * 64 + lane;
-        for (int m0 = 0; m0 < c; m0 += MT) {
-          float acc[MT];
-          dev::sum_slices<MT, 4>(
-              acc, [&](int s, int m) { return pt + (size_t(s) * n + pl.pos[min(m0 + m, c - 1)]) * 64; }, slices);
-#pragma unroll
-          for (int m = 0; m < MT; ++m)
-            if (m0 + m < c) finish(pl.pos[m0 + m], acc[m]);
+        for (int m = 0; m < c; ++m) {
+          float acc[1];
+          dev::sum_slices<1, 4>(acc, [&](int s, int) { return pt + (size_t(s) * n + pl.pos[m]) * 64; }, slices);
+          finish(pl.pos[m], acc[0]);
         }
         dev::reset_counter(ctr, lane);
       }
@@ -676,14 +662,14 @@ void launch_mm(const MoELaunch &a, const MoEGemm &mm, const MoEPlanSizes &p, hip
   hip_check(hipGetLastError(), "moe launch");
 }
 
-template <int MT, int GSW>
-void launch_mt(const MoELaunch &a, const MoEPlanSizes &p, hipStream_t s) {
+template <int GSW>
+void launch_k_moe(const MoELaunch &a, const MoEPlanSizes &p, hipStream_t s) {
   const int tgu = 2 * a.gu.blocks, tdn = a.dn.blocks;
   const int ggu = (tgu + 7) / 8 * 8 * p.slots * p.slices_gu;
   const int gdn = (tdn + 7) / 8 * 8 * p.slots * p.slices_dn;
   hipLaunchKernelGGL(k_moe_plan, dim3(p.slots + 1), dim3(64), 0, s, a, MoEGemm(), p.slots);
-  hipLaunchKernelGGL((k_moe<MT, GSW, false>), dim3(ggu), dim3(256), p.lds_gu, s, a, p.slices_gu, p.sps_gu, p.slots);
-  hipLaunchKernelGGL((k_moe<MT, GSW, true>), dim3(gdn), dim3(256), p.lds_dn, s, a, p.slices_dn, p.sps_dn, p.slots);
+  hipLaunchKernelGGL((k_moe<GSW, false>), dim3(ggu), dim3(256), p.lds_gu, s, a, p.slices_gu, p.sps_gu, p.slots);
+  hipLaunchKernelGGL((k_moe<GSW, true>), dim3(gdn), dim3(256), p.lds_dn, s, a, p.slices_dn, p.sps_dn, p.slots);
 }
 
 // ---- one token, one launch -----------------------------------------------
@@ -981,28 +967,25 @@ MoEPlanSizes moe_plan(const MoELaunch &a) {
   MoEPlanSizes p;
   const int n = a.rows * a.topk;
   p.slots = std::min(a.experts, n);
-  // One token per pass (one token in all, unless the matrix-core launches are
-  // turned off).
-  p.mt = 1;
   // Steps per wave: 8.  One row with its routes given would take 4 (13.36
   // against 13.63 us), but the launch that computes the routes itself is
   // faster at 8 (16.55 against 17.91 us) and must sum in the same order as the
   // routes-given launch, so one row keeps 8.  QNN_MOE_SPS overrides.
   // Bounded by the activation-slice LDS budget.
   const int forced = tuning().moe_sps;
-  auto steps = [&](const I4Layout &l, int) {
-    const int lds_cap = int((48 << 10) / (size_t(p.mt) * 4 * l.lanes * (dev::kXWords * 4 + 8)));
+  auto steps = [&](const I4Layout &l) {
+    const int lds_cap = int((48 << 10) / (size_t(4) * l.lanes * (dev::kXWords * 4 + 8)));
     const int cap = std::max(1, std::min(8, lds_cap));
     return std::min(forced > 0 ? forced : 8, cap);
   };
-  p.sps_gu = steps(a.gu, 2 * a.gu.blocks);
-  p.sps_dn = steps(a.dn, a.dn.blocks);
+  p.sps_gu = steps(a.gu);
+  p.sps_dn = steps(a.dn);
   p.slices_gu = (a.gu.steps + 4 * p.sps_gu - 1) / (4 * p.sps_gu);
   p.slices_dn = (a.dn.steps + 4 * p.sps_dn - 1) / (4 * p.sps_dn);
   const int need = std::max(p.sps_gu, p.sps_dn);
   p.gsw = need <= 1 ? 1 : (need <= 2 ? 2 : (need <= 4 ? 4 : 8));
-  p.lds_gu = dev::xplanes_bytes(p.mt, 4 * p.sps_gu * a.gu.lanes);
-  p.lds_dn = dev::xplanes_bytes(p.mt, 4 * p.sps_dn * a.dn.lanes);
+  p.lds_gu = dev::xplanes_bytes(1, 4 * p.sps_gu * a.gu.lanes);
+  p.lds_dn = dev::xplanes_bytes(1, 4 * p.sps_dn * a.dn.lanes);
   const int tgu = 2 * a.gu.blocks, tdn = a.dn.blocks;
   p.partial_floats = std::max(size_t(tgu) * p.slices_gu, size_t(tdn) * p.slices_dn) * n * 64;
   p.counters = (size_t(std::max(tgu, tdn)) * p.slots + tdn) * kCounterStride;
@@ -1038,11 +1021,11 @@ bool moe_gemm_applies(const MoELaunch &a) {
 }
 
 void moe_launch(const MoELaunch &a, const MoEPlanSizes &p, hipStream_t s) {
-  switch (p.mt * 16 + p.gsw) {
-    case 1 * 16 + 1: launch_mt<1, 1>(a, p, s); break;
-    case 1 * 16 + 2: launch_mt<1, 2>(a, p, s); break;
-    case 1 * 16 + 4: launch_mt<1, 4>(a, p, s); break;
-    case 1 * 16 + 8: launch_mt<1, 8>(a, p, s); break;
+  switch (p.gsw) {
+    case 1: launch_k_moe<1>(a, p, s); break;
+    case 2: launch_k_moe<2>(a, p, s); break;
+    case 4: launch_k_moe<4>(a, p, s); break;
+    case 8: launch_k_moe<8>(a, p, s); break;
     default: fail(QNN_E_INVALID_OP, "MoE launch plan");
   }
   hip_check(hipGetLastError(), "moe launch");
@@ -1050,7 +1033,7 @@ void moe_launch(const MoELaunch &a, const MoEPlanSizes &p, hipStream_t s) {
 
 MoEDecodePlan moe_decode_plan(const MoELaunch &a, const MoEPlanSizes &p) {
   MoEDecodePlan d;
-  if (a.rows != 1 || p.mt != 1 || a.gu.lanes != 1 || a.dn.lanes != 1 || p.sps_gu != p.sps_dn) return d;
+  if (a.rows != 1 || a.gu.lanes != 1 || a.dn.lanes != 1 || p.sps_gu != p.sps_dn) return d;
   if (p.gsw != 1 && p.gsw != 2 && p.gsw != 4 && p.gsw != 8) return d;
   const int k = a.topk;
   const int pairs = k * a.gu.blocks;
