@@ -463,8 +463,10 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
 // * down (<.., true>): a workgroup is four blocks, two waves (K-halves) each.
 // * k_moe_combine adds a token's experts in ascending id, as k_moe does.
 // The next chunk's weights (four groups) are requested before the current
-// chunk's products; more comes from the four waves per SIMD (a wave's scales
-// go through LDS: as four loads per lane they took 128 registers and spilled).
+// chunk's products, but the activations of the chunk's groups 1 to 3 after
+// them, and loads return in order: a wave waits for those weights once a chunk,
+// and it is the other three waves of the SIMD that hide it.  (A wave's scales
+// go through LDS: as four loads per lane they took 128 registers and spilled.)
 //
 // Measured, whole layer with router and route, 128 experts of 768 x 2048, top
 // 8: 128 tokens 525 -> 129 us (338 with the router's share gone; gate/up 69
