@@ -30,9 +30,11 @@
 // x channels) and read by its four waves, 32 query rows each; the next tile's
 // elements are on their way to registers meanwhile.
 //
-// What bounds it: per 64 keys and wave 96 MFMAs (18.5 ns each) against about
-// 1000 VALU operations (softmax, planes of p, a share of the planes of K and
-// V), which two waves per SIMD run under each other's products.  At dim 128
+// What bounds it: the VALU (softmax, planes of w, a share of the planes of K and
+// V).  Counters, 128 rows over 4096 keys: 17 VALU operations per MFMA, so per 64
+// keys and wave 1640 of 4 cycles against 96 MFMAs of 32, which two waves per
+// SIMD run under each other's products; VALU busy 49 % and matrix cores 19 % of
+// the elapsed cycles, waves waiting 26 % of theirs.  At dim 128
 // that takes tiles of 32 keys (236 registers; 64 keys do not fit two waves per
 // SIMD).  A KV head's keys are split over two workgroups per CU; k_attn_merge
 // joins the parts.  Infinities and NaNs among a workgroup's keys or query rows

@@ -22,10 +22,13 @@
 // Measured against 64 bits the products are an order of magnitude closer than
 // the matvec's (1e-7 of the result against 1e-5).
 //
-// What bounds it: the matrix cores (two fp16 planes: 4 M N K operations; a
-// SIMD retires one of these MFMAs in 18.5 ns, so a K-tile of 128 x 128 outputs
-// takes 0.59 us at least and 0.85 us as built), then the ends of a workgroup
-// (first loads, group halves, partial sums: 4.4 us).  Hence:
+// What bounds it: no unit alone.  The matrix cores have 4 M N K operations (two
+// fp16 planes; a SIMD of a full card retires one of these MFMAs in 18.5 ns, so a
+// K-tile of 128 x 128 outputs takes 0.59 us at least and 0.85 us as built), and
+// the ends of a workgroup (first loads, group halves, partial sums) take 4.4 us.
+// Counters, gate/up pair at 128 rows: matrix cores busy 24 %, VALU (folds,
+// unpacking) 31 % of the elapsed cycles, waves waiting 29 % of theirs; 38 MB read
+// for 31 of weights, 30 MB of partial sums written.  Hence:
 // * a workgroup is eight waves, two per SIMD, so that one's folds run under
 //   the other's products: 2 (rows) x 2 (weight blocks of 64 rows) x 2 (the
 //   two groups of a K-tile), the group halves meeting in LDS at the end;

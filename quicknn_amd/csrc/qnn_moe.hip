@@ -452,8 +452,10 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
 // tiles, v_mfma_f32_16x16x32_f16 taking a whole group of 16 tokens x 16 weight
 // rows.  Every routed weight is unpacked once for up to 16 TT tokens, where
 // k_moe makes a pass of 16 v_dot4 and a staging barrier per token (gate/up
-// 185 us, down 147 us at that chunk).  What bounds it is the weight stream;
-// per 64 x 32 weights the VALU has 56 operations.
+// 185 us, down 147 us at that chunk).  What bounds it is the weight stream:
+// counters, gate/up at 128 tokens, 316 MB in 67 us, the rate of a large copy (the
+// weights are 252 MB: a wave's last chunk, of four, is requested twice); VALU
+// busy 40 %, matrix cores 15 %.
 // * the planning launch prepares the token rows too, k_moe_act the h rows
 //   between the launches.  Pieces are row-major, so a lane gathers its token's
 //   piece from wherever the row is.
@@ -469,8 +471,8 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
 // go through LDS: as four loads per lane they took 128 registers and spilled.)
 //
 // Measured, whole layer with router and route, 128 experts of 768 x 2048, top
-// 8: 128 tokens 525 -> 129 us (338 with the router's share gone; gate/up 69
-// us, 3.6 TB/s, down 43 us), 32 tokens 309 -> 105, 8 tokens 183 -> 66, 2
+// 8: 128 tokens 525 -> 127 us (338 with the router's share gone; gate/up 67
+// us, down 39 us), 32 tokens 309 -> 105, 8 tokens 183 -> 66, 2
 // tokens 141 -> 41 us; 8 experts of 256 x 512, top 2, 2 tokens 43 -> 32 us:
 // faster from two tokens on at every shape measured, so from two.
 __global__ __launch_bounds__(256) void k_moe_act(const float *__restrict__ x, int rows, int K, int gpad,
