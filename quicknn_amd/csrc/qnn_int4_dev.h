@@ -607,9 +607,27 @@ __device__ __forceinline__ half8 unpack_i4(uint32_t w, const I4Masks &mk) {
   return r;
 }
 
-// An activation row's planes: v = x 2^-e (exact), hi = fp16(v), lo = fp16(v -
-// hi); an infinity or NaN is in hi alone.  act_exp: the row's e from its
-// largest magnitude; below 2^-110 rows keep that scale, which stays finite.
+// The same times 2^-11, for the lower plane below (exact).
+__device__ __forceinline__ half8 lower_i4(const half8 &w) {
+  const half2v f = {_Float16(0.00048828125f), _Float16(0.00048828125f)};
+  half2v v[4];
+  __builtin_memcpy(v, &w, 16);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] *= f;
+  half8 r;
+  __builtin_memcpy(&r, v, 16);
+  return r;
+}
+
+// An activation row's planes: v = x 2^-e (exact), hi = fp16(v), lo = fp16((v -
+// hi) 2^11), whose products take lower_i4's weights; an infinity or NaN is in hi
+// alone.  With its own factor lo has the range of hi: 22 bits of every element
+// down to 2^-27 of its row's largest, and 2^-49 of that largest below (without,
+// 2^-17 and 2^-38).  The fixed point of the matvec has 16 bits per group of 32,
+// and a group of weights may be zero where the row's largest element is.
+// (Four MLP layers of 2560 -> 9728 at 128 rows 355 -> 362 us for it.)
+// act_exp: the row's e from its largest magnitude; below 2^-110 rows keep that
+// scale, which stays finite.
 __device__ __forceinline__ int act_exp(float amax) { return max(range_exp(amax), -110); }
 // 8 elements -> two pieces of 8 halfs in unpack_i4's order.
 __device__ __forceinline__ void act_planes(const float (&x)[8], float scale, uint4 &ph, uint4 &pl) {
@@ -618,7 +636,7 @@ __device__ __forceinline__ void act_planes(const float (&x)[8], float scale, uin
   for (int i = 0; i < 8; ++i) {
     const float s = x[i] * scale;
     hi[i] = float(_Float16(s));
-    lo[i] = isfinite(hi[i]) ? s - hi[i] : 0.0f;
+    lo[i] = isfinite(hi[i]) ? (s - hi[i]) * 2048.0f : 0.0f;
   }
   ph = make_uint4(pack_h2(hi[0], hi[4]), pack_h2(hi[1], hi[5]), pack_h2(hi[2], hi[6]), pack_h2(hi[3], hi[7]));
   pl = make_uint4(pack_h2(lo[0], lo[4]), pack_h2(lo[1], lo[5]), pack_h2(lo[2], lo[6]), pack_h2(lo[3], lo[7]));

@@ -9,7 +9,7 @@
 //     C[m][n] = sum_g s[n][g] * sum_{k in group g} x[m][k] (q[n][k] - 8)
 //
 // * x is prepared once per call (k_i4_act): scaled per row by a power of two
-//   and split into two fp16 values, hi = fp16(x'), lo = fp16(x' - hi): 22
+//   and split into two fp16 values, hi = fp16(x'), lo = fp16((x' - hi) 2^11): 22
 //   significant bits, against the 16 bits of the matvec's fixed point.
 // * q - 8 is an exact fp16 integer, unpacked in registers: nibbles under the
 //   exponent of 1024, then one packed fp16 add or fma (9 operations for 8
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(512) void k_i4_gemm(const I4GemmArgs a) {
       d[0][t][e] = d[1][t][e] = 0.0f;
     }
   half8 af[MB][2][2];  // [row block][plane][kk]
-  half8 bf[2][2][2];   // [K-tile parity][32-row half of the block][kk]
+  half8 bf[2][2][2][2];  // [K-tile parity][32-row half of the block][plane][kk]
   float sc[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};  // [K-tile parity][32-row half]
 
   auto stage_at = [&](int kt) { return reinterpret_cast<const uint8_t *>(lds) + uint32_t(kt % SG::ST) * SG::BYTES; };
@@ -253,10 +253,13 @@ __global__ __launch_bounds__(512) void k_i4_gemm(const I4GemmArgs a) {
     f[1] = s[128];
   };
   // Row l's dwords (lane l) -> dword 2h + kk of row 32 t + lane % 32 (h = lane / 32).
-  auto unpack_pair = [&](half8 (&f)[2][2], uint32_t d0, uint32_t d2, int kk) {
+  auto unpack_pair = [&](half8 (&f)[2][2][2], uint32_t d0, uint32_t d2, int kk) {
     const auto r = __builtin_amdgcn_permlane32_swap(d0, d2, false, false);
-    f[0][kk] = dev::unpack_i4(r[0], masks);
-    f[1][kk] = dev::unpack_i4(r[1], masks);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f[t][0][kk] = dev::unpack_i4(r[t], masks);
+      f[t][1][kk] = dev::lower_i4(f[t][0][kk]);
+    }
   };
 
   // One K-tile (P: its parity).  Phase i runs the 8 MFMAs of row block i, two
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(512) void k_i4_gemm(const I4GemmArgs a) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int t = j & 1, p = j >> 2, kk = (j >> 1) & 1;
-        d[D][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][p][kk], bf[P][t][kk], j < 2 ? zero : d[D][t], 0, 0, 0);
+        d[D][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][p][kk], bf[P][t][p][kk], j < 2 ? zero : d[D][t], 0, 0, 0);
         if (j < 4) {
           if (MB == 2) read_a(af[i ^ 1], i == 0 ? st0 : st1, i ^ 1, j);
           else read_a(an, st1, 0, j);

@@ -556,21 +556,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TT == 1 ? 4
         dev::half8 bw[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) bw[r] = dev::unpack_i4(wq[r], masks);
+        f32x4 s[TT][4];
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
-          dev::half8 xh, xl;
+          dev::half8 xh;
           __builtin_memcpy(&xh, &xa[g & 1][t][0], 16);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            s[t][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, bw[r], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // in place: both at once do not fit the registers of four waves
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bw[r] = dev::lower_i4(bw[r]);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          dev::half8 xl;
           __builtin_memcpy(&xl, &xa[g & 1][t][1], 16);
-          f32x4 s[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            s[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, bw[r], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, bw[r], s[r], 0, 0, 0);
+          for (int r = 0; r < 4; ++r) s[t][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, bw[r], s[t][r], 0, 0, 0);
 #pragma unroll
           for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[t][r][i] = fmaf(s[r][i], sc[r], acc[t][r][i]);
+            for (int i = 0; i < 4; ++i) acc[t][r][i] = fmaf(s[t][r][i], sc[r], acc[t][r][i]);
         }
         __builtin_amdgcn_sched_barrier(0);  // one group's unpacked weights at a time
       }

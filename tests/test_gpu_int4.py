@@ -334,3 +334,27 @@ def test_many_rows_gemm(ctx, rng, rows, n, k):
         assert np.array_equal(ctx.Download(dst).view(np.uint32), got.view(np.uint32))
     for t in (src, dst, few, half):
         ctx.Recycle(t)
+
+
+@pytest.mark.parametrize("rows", [25, 100])
+@pytest.mark.parametrize("large", [1e7, 1e8, 1e10])
+def test_many_rows_gemm_large_element_under_zero_weights(ctx, rng, rows, large):
+    """A group of weights may be zero (scale 0) where an activation row has its largest element, which then has no part
+    in the result: the row's other elements keep 22 bits down to 2^-27 of it, and 2^-49 of it below, so the bound is
+    test_many_rows_gemm's with that step (the matvec's fixed point has 16 bits of each group's own largest)."""
+    n, k = 200, 256
+    p = make_int4(rng, n, k)
+    p.reshape(n, k // 32, 20)[:, 1, :4] = 0
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[::2, 40] = large
+    x[1::2, 63] = -large
+    w = hip.MemoryBlock.int4(p)
+    src, dst = ctx.UploadRaw(x), ctx.NewTensor(rows * n)
+    ctx.Int4Linear(dst, src, w, rows, k, n)
+    got = ctx.Download(dst).reshape(rows, n)
+    w64, x64 = oracle.int4_dequant(p, k).astype(np.float64), x.astype(np.float64)
+    bound = (np.abs(x64) @ np.abs(w64).T) * (2.0 ** -21 + (64 + k / 32) * 2.0 ** -24)
+    bound += np.abs(x64).max(1)[:, None] * 2.0 ** -49 * np.abs(w64).sum(1)
+    assert np.all(np.abs(got - x64 @ w64.T) <= bound)
+    for t in (src, dst):
+        ctx.Recycle(t)

@@ -431,3 +431,29 @@ def test_moe_experts_matrix_core_launches(ctx, rng, tune, E, hidden, inter, k, r
     for r in range(rows):
         assert normwise_rel_err(mm[r], dot[r]) <= 2e-4, r
         assert normwise_rel_err(mm[r], want[r]) <= TOL, r
+
+
+@pytest.mark.parametrize("E,hidden,inter,k,rows", [(4, 256, 128, 2, 3), (2, 128, 64, 1, 100)])
+def test_moe_matrix_core_large_element_under_zero_weights(ctx, rng, tune, E, hidden, inter, k, rows):
+    """A token's largest element where every routed expert's gate and up weights are zero (scale 0) takes no bits from
+    its other elements: 2^-49 of 1e9 is 2e-6 of them, below the 16 bits per group of the dot kernel, so the two agree
+    as in test_moe_experts_matrix_core_launches."""
+    ex = Experts(rng, E, hidden, inter)
+    for p in ex.g + ex.u:
+        p.reshape(inter, hidden // 32, 20)[:, 1, :4] = 0
+    s = ctx.CreateExpertSet(ex.bg, ex.bu, ex.bd, hidden, inter)
+    x = rng.standard_normal((rows, hidden)).astype(np.float32)
+    x[:, 40] = 1e9
+    routes, ids, probs = route_on_gpu(ctx, rng.standard_normal((rows, E)).astype(np.float32), k)
+    src, dst, got = ctx.UploadRaw(x), ctx.NewTensor(rows * hidden), {}
+    for name, frm in (("mm", "2"), ("dot", "0")):
+        tune("QNN_MOE_GEMM_ROWS", frm)
+        ctx.MoEExperts(s, dst, src, routes, rows, k)
+        got[name] = ctx.Download(dst).reshape(rows, hidden)
+    ctx.DestroyExpertSet(s)
+    want = ex.oracle(x, ids, probs)
+    for r in range(rows):
+        assert normwise_rel_err(got["mm"][r], got["dot"][r]) <= 2e-4, r
+        assert normwise_rel_err(got["mm"][r], want[r]) <= TOL, r
+    for t in (src, dst):
+        ctx.Recycle(t)
