@@ -38,8 +38,10 @@
 // that takes tiles of 32 keys (236 registers; 64 keys do not fit two waves per
 // SIMD).  A KV head's keys are split over two workgroups per CU; k_attn_merge
 // joins the parts.  Infinities and NaNs among a workgroup's keys or query rows
-// send its part to a plain loop over its rows, since 0 times them would reach
-// rows that do not see the key, and NaN where the score is infinite.
+// send its part to a plain fp32 loop over its rows, four per wave, since 0 times
+// them would reach rows that do not see the key, and NaN where the score is
+// infinite.  (128 rows over 4096 keys with one hidden NaN: 1.05 ms, a row per
+// wave and a key at a time 5.4; k_attn 0.46.)
 // More than 128 channels stay with k_attn: at 256 the output of 32 rows (128
 // registers) and the planes of q (128) are all that a wave of two per SIMD has.
 //
@@ -565,41 +567,80 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // Infinities or NaNs among the keys would reach rows that do not see them
     // through the products' zeros, and in q would meet the zeros of the lower
     // planes (inf, which a soft cap makes finite, would be NaN): this part is
-    // computed row by row instead, a wave per query row, in fp32 as k_attn does.
-    for (int i = wave; i < kQRows && q0 + i < nq; i += 4) {
-      const int row = (q0 + i) / a.group, hd = kh * a.group + (q0 + i) % a.group;
-      const float *qr = a.q + (size_t(row) * a.heads + hd) * a.dim;
-      const unsigned *mrow =
-          reinterpret_cast<const unsigned *>(a.cache + 2 * size_t(a.cap) * width) + size_t(row) * a.cap;
-      const float mul = a.scale > 0.0f ? a.scale : 1.0f / sqrtf(float(a.dim));
-      float m = -INFINITY, l = 0.0f, o[2] = {0.0f, 0.0f};  // channels lane, lane + 64
-      for (int key = max(first_key(row), tb * KT); key < min(a.position + row + 1, te * KT); ++key) {
-        if (a.masked && mrow[key] == 0u) continue;
-        float d = 0.0f;
-        for (int c = lane; c < a.dim; c += 64) d += qr[c] * kt[size_t(c) * a.cap + key];
-        float sc = dev::wave_sum_xor(d) * mul;
-        if (a.softcap > 0.0f) sc = a.softcap * tanhf(fminf(fmaxf(sc / a.softcap, -20.0f), 20.0f));
-        const float mn = fmaxf(m, sc);
-        // (a NaN before any other key counts, too)
-        const float kp = mn == -INFINITY ? 1.0f : expf(m - mn), w = sc == -INFINITY ? 0.0f : expf(sc - mn);
-        l = l * kp + w;
-        m = mn;
-        for (int c = lane, j = 0; c < a.dim; c += 64, ++j) {
-          const float add = w * vb[size_t(key) * a.dim + c];
-          if (j == 0) o[0] = o[0] * kp + add;
-          else o[1] = o[1] * kp + add;
+    // computed in fp32 as k_attn does, a wave per four query rows: a lane per key
+    // for the scores, per channel for the values.
+    constexpr int R = 4;
+    const float mul = a.scale > 0.0f ? a.scale : 1.0f / sqrtf(float(a.dim));
+    const unsigned *m0 = reinterpret_cast<const unsigned *>(a.cache + 2 * size_t(a.cap) * width);
+    const int c0 = min(lane, a.dim - 1), c1 = min(lane + 64, a.dim - 1);
+    for (int i = R * wave; i < kQRows && q0 + i < nq; i += 4 * R) {
+      int row[R];
+      size_t rh[R];
+      float m[R], l[R], o[R][2];  // channels lane, lane + 64
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        const int x = min(q0 + i + j, nq - 1);
+        row[j] = x / a.group;
+        rh[j] = size_t(row[j]) * a.heads + kh * a.group + x % a.group;
+        m[j] = -INFINITY;
+        l[j] = o[j][0] = o[j][1] = 0.0f;
+      }
+      const int first = max(first_key(row[0]), tb * KT), end = min(a.position + row[R - 1] + 1, te * KT);
+      for (int k0 = first; k0 < end; k0 += 64) {
+        const int key = min(k0 + lane, end - 1);
+        float d[R], w[R];
+        uint64_t seen[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) d[j] = 0.0f;
+#pragma unroll 8
+        for (int c = 0; c < a.dim; ++c) {
+          const float kv = kt[size_t(c) * a.cap + key];
+#pragma unroll
+          for (int j = 0; j < R; ++j) d[j] += a.q[rh[j] * a.dim + c] * kv;
+        }
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          bool ok = k0 + lane < end && key >= first_key(row[j]) && key <= a.position + row[j];
+          if (ok && a.masked) ok = m0[size_t(row[j]) * a.cap + key] != 0u;
+          float sc = d[j] * mul;
+          if (a.softcap > 0.0f) sc = a.softcap * tanhf(fminf(fmaxf(sc / a.softcap, -20.0f), 20.0f));
+          const float mn = fmaxf(m[j], dev::wave_max_xor(ok ? sc : -INFINITY));
+          const float kp = mn == -INFINITY ? 1.0f : expf(m[j] - mn);
+          w[j] = ok && sc != -INFINITY ? expf(sc - mn) : 0.0f;  // (a NaN before any other key counts, too)
+          l[j] = l[j] * kp + dev::wave_sum_xor(w[j]);
+          m[j] = mn;
+          o[j][0] *= kp;
+          o[j][1] *= kp;
+          seen[j] = __ballot(ok);
+        }
+        for (int u0 = 0; u0 < min(64, end - k0); u0 += 8) {
+#pragma unroll
+          for (int u = u0; u < u0 + 8; ++u) {
+            const float *v = vb + size_t(min(k0 + u, end - 1)) * a.dim;
+            const float v0 = v[c0], v1 = v[c1];
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+              const float wu = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w[j]), u));
+              const bool see = (seen[j] >> u) & 1u;  // what the row does not see may be anything
+              const float a0 = wu * v0, a1 = wu * v1;
+              o[j][0] += see ? a0 : 0.0f;
+              o[j][1] += see ? a1 : 0.0f;
+            }
+          }
         }
       }
-      const size_t rh = size_t(row) * a.heads + hd;
-      float *dst = a.splits == 1 ? a.out + rh * a.dim : a.opart + (size_t(split) * a.rows * a.heads + rh) * a.dim;
-      for (int c = lane, j = 0; c < a.dim; c += 64, ++j) {
-        const float v = j == 0 ? o[0] : o[1];
-        dst[c] = a.splits == 1 ? v / l : v;
-      }
-      if (a.splits > 1 && lane == 0) {
-        float *ml = a.ml + (size_t(split) * a.rows * a.heads + rh) * 2;
-        ml[0] = m;
-        ml[1] = l;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        if (q0 + i + j >= nq) continue;
+        const bool whole = a.splits == 1;
+        float *dst = whole ? a.out + rh[j] * a.dim : a.opart + (size_t(split) * a.rows * a.heads + rh[j]) * a.dim;
+        if (lane < a.dim) dst[lane] = whole ? o[j][0] / l[j] : o[j][0];
+        if (lane + 64 < a.dim) dst[lane + 64] = whole ? o[j][1] / l[j] : o[j][1];
+        if (!whole && lane == 0) {
+          float *ml = a.ml + (size_t(split) * a.rows * a.heads + rh[j]) * 2;
+          ml[0] = m[j];
+          ml[1] = l[j];
+        }
       }
     }
     return;

@@ -434,6 +434,36 @@ def test_attention_of_many_rows_infinite_keys(ctx, rng, tune, where, value):
         ctx.Recycle(z)
 
 
+@pytest.mark.parametrize("dim", [33, 64, 80, 128])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_attention_of_many_rows_hidden_infinities(ctx, rng, tune, dim, value):
+    """Infinities and NaNs in keys that the mask hides: the part that holds them is computed row by row, each row as if
+    they were not there, in chunks of 64 keys (parts of one chunk and of several, a chunk that starts with such a key)."""
+    rows, heads, kvh, cap, pos = 48, 8, 2, 420, 360
+    q, cache = many_inputs(rng, (rows, heads, kvh, dim, cap, pos, 0, 0.0, 0.0, True))
+    hidden = (0, 64, 200, 201, 390)
+    kt, vs = cache[:kvh * dim * cap].reshape(kvh, dim, cap), cache[kvh * dim * cap:2 * kvh * dim * cap].reshape(kvh, cap, dim)
+    m = cache.view(np.uint32)[2 * cap * kvh * dim:].reshape(rows, cap)
+    for key in hidden:
+        kt[:, :, key] = value
+        vs[:, key] = value
+        m[:, key] = 0
+    m[np.arange(rows), pos + np.arange(rows)] = 1
+    kt[:, :, 390] = vs[:, 390] = 1.0  # row 30's own key
+    want = oracle.cached_attention(q, cache, rows, cap, heads, kvh, dim, pos, 0, 0.0, 0.0, True).reshape(rows * heads, dim)
+    assert np.all(np.isfinite(want))
+    tq, tc, to = up(ctx, q), up(ctx, cache), ctx.NewTensor(rows * heads * dim)
+    tune("QNN_ATTN_MM", "1")
+    for wgs in ("512", "1"):
+        tune("QNN_ATTN_WGS", wgs)
+        ctx.CachedAttention(to, tq, tc, rows, cap, heads, kvh, dim, pos, 0, 0.0, 0.0, True)
+        got = ctx.Download(to).reshape(rows * heads, dim)
+        for i in range(rows * heads):
+            assert normwise_rel_err(got[i], want[i]) <= 1e-5, (wgs, i)
+    for z in (tq, tc, to):
+        ctx.Recycle(z)
+
+
 @pytest.mark.parametrize("softcap", [0.0, 30.0])
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
 def test_attention_of_many_rows_infinite_queries(ctx, rng, tune, value, softcap):
