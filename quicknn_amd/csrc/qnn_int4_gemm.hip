@@ -26,8 +26,8 @@
 // fp16 planes; a SIMD of a full card retires one of these MFMAs in 18.5 ns, so a
 // K-tile of 128 x 128 outputs takes 0.59 us at least and 0.85 us as built), and
 // the ends of a workgroup (first loads, group halves, partial sums) take 4.4 us.
-// Counters, gate/up pair at 128 rows: matrix cores busy 24 %, VALU (folds,
-// unpacking) 31 % of the elapsed cycles, waves waiting 29 % of theirs; 38 MB read
+// Counters, gate/up pair at 128 rows: matrix cores busy 23 %, VALU (folds,
+// unpacking) 32 % of the elapsed cycles, waves waiting 29 % of theirs; 38 MB read
 // for 31 of weights, 30 MB of partial sums written.  Hence:
 // * a workgroup is eight waves, two per SIMD, so that one's folds run under
 //   the other's products: 2 (rows) x 2 (weight blocks of 64 rows) x 2 (the
@@ -44,9 +44,9 @@
 // one launch.
 //
 // Measured, 128 rows, weights rotated beyond the caches: gate/up pair of 2560
-// -> 9728 36 us + 8 us of sums and 5 us of activations (the matvec kernels:
-// 8 launches of 19 us), down 9728 -> 2560 19 + 5 + 7 us (8 x 12 us); a whole
-// MLP layer with its norm and residual 259 -> 86 us, at 64 rows 135 -> 66, at
+// -> 9728 39 us + 9 us of sums and 5 us of activations (the matvec kernels:
+// 8 launches of 19 us), down 9728 -> 2560 21 + 6 + 8 us (8 x 12 us); a whole
+// MLP layer with its norm and residual 259 -> 90 us, at 64 rows 135 -> 66, at
 // 32 rows 73 -> 63 us.  K-slices of that pair: 1 51.5 us, 2 55.7, 3 49.2, 4
 // 56.5, 5 54.6; of that down: 6 39.5, 8 36.3, 10 33.5, 12 34.2, 13 44.3 us.
 // From how many rows (Tuning::i4_gemm_rows): an MLP layer at 17 rows takes

@@ -453,9 +453,9 @@ __global__ __launch_bounds__(256) void k_moe(const MoELaunch a, const int slices
 // rows.  Every routed weight is unpacked once for up to 16 TT tokens, where
 // k_moe makes a pass of 16 v_dot4 and a staging barrier per token (gate/up
 // 185 us, down 147 us at that chunk).  What bounds it is the weight stream:
-// counters, gate/up at 128 tokens, 316 MB in 67 us, the rate of a large copy (the
+// counters, gate/up at 128 tokens, 314 MB in 65 us, the rate of a large copy (the
 // weights are 252 MB: a wave's last chunk, of four, is requested twice); VALU
-// busy 40 %, matrix cores 15 %.
+// busy 51 %, matrix cores 16 % of the elapsed cycles.
 // * the planning launch prepares the token rows too, k_moe_act the h rows
 //   between the launches.  Pieces are row-major, so a lane gathers its token's
 //   piece from wherever the row is.
