@@ -701,7 +701,8 @@ bool attn_mm_plan(AttnPlan &p, int rows, int cap, int heads, int kv_heads, int d
   const int last_end = position + rows;
   const long long least = ((long long)min_k << 10) * (dim > 64 && dim <= 96 ? 5 : 4) / 4;
   if (min_k <= 0 || rows < 4 || dim > 128 || nq > (1 << 24) ||
-      size_t(dim) * cap * 4 > 0x7FFFFFFFull ||  // 32-bit offsets within a KV head
+      // 32-bit offsets within a KV head, those of dims past the last (up to 64 or 128) included
+      size_t(dim) * cap * 4 > 0x7FFFFFFFull || size_t(dim <= 64 ? 64 : 128) * (size_t(cap) + 64) * 4 > 0xFFFFFFFFull ||
       (long long)rows * heads * (window > 0 ? std::min(window, last_end) : last_end) < least)
     return false;
   p.qtiles = int((nq + kQRows - 1) / kQRows);
